@@ -1271,32 +1271,6 @@ size_t attention_workspace_floats(int heads, int max_chunks, int head_dim)
     return size_t(heads) * size_t(max_chunks) * size_t(head_dim + 2);
 }
 
-// One chunk per block: the most blocks in flight (1024 positions: 13.6 us
-// against 25.5 us with four chunks per block, 4096: 25.9 against 33.2).
-constexpr int kChunksPerBlock = 1;
-
-int attention_splits(int context)
-{
-    const int nc = (context + kAttnChunk - 1) / kAttnChunk;
-    return (nc + kChunksPerBlock - 1) / kChunksPerBlock;
-}
-
-template <int D, int GMAX, bool STEP>
-static hipError_t launch_attn(const AttnParams& a, hipStream_t s)
-{
-    const int batch = (!STEP && a.batch > 1) ? a.batch : 1;
-    const int splits = (a.max_chunks + kChunksPerBlock - 1) / kChunksPerBlock;
-    hipLaunchKernelGGL((attention_kernel<D, GMAX, STEP, kChunksPerBlock>), dim3(a.kv_heads, splits, batch),
-                       dim3(kBlock), 0, s, a);
-    if (a.max_chunks > 1) {
-        constexpr int hpb = kBlock / D;
-        const int heads = a.kv_heads * a.groups;
-        hipLaunchKernelGGL((attention_combine_kernel<D, STEP>), dim3((heads + hpb - 1) / hpb, batch), dim3(kBlock),
-                           0, s, a);
-    }
-    return hipGetLastError();
-}
-
 hipError_t launch_batch_attention(const AttnParams& a, hipStream_t s)
 {
     if (a.head_dim != 128 || !a.table || !a.qkv || !a.q8 || !a.act || a.groups > 8 ||
@@ -1387,22 +1361,38 @@ hipError_t launch_batch_qkv_attention(const int8_t* x, const float* act, const u
     return hipGetLastError();
 }
 
-hipError_t launch_attention(const AttnParams& a, bool step_mode, hipStream_t s)
+// The step's attention: one chunk per block, the most blocks in flight
+// (1024 positions: 13.6 us against 25.5 us with four chunks per block, 4096:
+// 25.9 against 33.2).
+hipError_t launch_step_attention(const AttnParams& a, hipStream_t s)
 {
-    if (step_mode) {
-        if (a.head_dim != 128 || a.groups > 4) return hipErrorInvalidValue;
-        return launch_attn<128, 4, true>(a, s);
+    if (a.head_dim != 128 || a.groups > 4) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((attention_kernel<128, 4, true, 1>), dim3(a.kv_heads, a.max_chunks), dim3(kBlock), 0, s, a);
+    if (a.max_chunks > 1) {
+        const int hpb = kBlock / 128;
+        hipLaunchKernelGGL((attention_combine_kernel<128, true>), dim3((a.kv_heads * a.groups + hpb - 1) / hpb),
+                           dim3(kBlock), 0, s, a);
     }
-    switch (a.head_dim) {
-    case 16: return launch_attn<16, 8, false>(a, s);
-    case 32: return launch_attn<32, 8, false>(a, s);
-    case 64: return launch_attn<64, 8, false>(a, s);
-    case 128:
-        // up to four query heads per kv head (Qwen3-4B's 32/8): the V
-        // accumulation then runs two (head, dim) pairs per thread, not four
-        return a.groups <= 4 ? launch_attn<128, 4, false>(a, s) : launch_attn<128, 8, false>(a, s);
-    default: return hipErrorInvalidValue;
-    }
+    return hipGetLastError();
+}
+
+hipError_t launch_one_chunk_attention(const AttnParams& a, hipStream_t s)
+{
+    if (a.head_dim != 128 || a.context + a.batch - 1 > kAttnChunk) return hipErrorInvalidValue;
+    if (a.groups <= 4)
+        hipLaunchKernelGGL((attention_kernel<128, 4, false, 1>), dim3(a.kv_heads, 1, a.batch), dim3(kBlock), 0, s, a);
+    else
+        hipLaunchKernelGGL((attention_kernel<128, 8, false, 1>), dim3(a.kv_heads, 1, a.batch), dim3(kBlock), 0, s, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_attention_combine(const AttnParams& a, hipStream_t s)
+{
+    if (a.head_dim != 128) return hipErrorInvalidValue;
+    const int hpb = kBlock / 128;
+    hipLaunchKernelGGL((attention_combine_kernel<128, false>), dim3((a.kv_heads * a.groups + hpb - 1) / hpb, a.batch),
+                       dim3(kBlock), 0, s, a);
+    return hipGetLastError();
 }
 
 // ---- the drop-in GQA decode in one launch ------------------------------------------

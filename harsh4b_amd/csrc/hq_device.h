@@ -52,6 +52,28 @@ __device__ __forceinline__ float spec_expf(float x)
     return p;
 }
 
+// spec_expf for x <= 0 (or NaN), without branches: the exponent of e^x is
+// in [-126, 0] wherever x >= -87, so the two power-of-two multiplies are one
+// exact ldexp.
+__device__ __forceinline__ float spec_expf_neg(float x)
+{
+    const bool zero = x < -87.0f;
+    const float y = zero ? -87.0f : x;      // (NaN passes through)
+    const float n = __builtin_rintf(y * 0x1.715476p+0f);
+    float r = __builtin_fmaf(-n, 0x1.62e400p-1f, y);
+    r = __builtin_fmaf(-n, 0x1.7f7d1cp-20f, r);
+    float p = 0x1.a01a02p-13f;
+    p = __builtin_fmaf(p, r, 0x1.6c16c2p-10f);
+    p = __builtin_fmaf(p, r, 0x1.111112p-7f);
+    p = __builtin_fmaf(p, r, 0x1.555556p-5f);
+    p = __builtin_fmaf(p, r, 0x1.555556p-3f);
+    p = __builtin_fmaf(p, r, 0.5f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_ldexpf(p, int(n));
+    return zero ? 0.0f : p;
+}
+
 // fp16 storage (RNE on the way in, exact widening on the way out).
 __device__ __forceinline__ uint16_t f32_to_f16(float x)
 {

@@ -164,7 +164,31 @@ hipError_t gemm_run_tail(const int8_t* x, const float* act, const uint8_t* w, co
                          const GemmTail& tail, hipStream_t s);
 hipError_t gemm_run(const int8_t* x, const float* act, const uint8_t* w, const float* ws, float* out, int m, int n,
                     int k, char* scratch, hipStream_t s);
-hipError_t launch_attention(const AttnParams& a, bool step_mode, hipStream_t s);
+// The decode step's attention (q/k norms, RoPE, K/V write, attention).
+hipError_t launch_step_attention(const AttnParams& a, hipStream_t s);
+// a.batch queries of one chunk at most (query z attends a.context + z
+// positions), one block per query and kv head.
+hipError_t launch_one_chunk_attention(const AttnParams& a, hipStream_t s);
+// The combine of the chunk partials in a.part for a.batch queries, query z
+// attending a.context + z positions (one-chunk queries are left alone).
+hipError_t launch_attention_combine(const AttnParams& a, hipStream_t s);
+
+// ---- prompt attention (hq_prefill_attn.hip) ---------------------------------------
+struct PrefillAttnParams {
+    const float* q;             // [rows, heads, 128], normed and rotated
+    uint16_t* keys;             // this layer's cache, rows up to p0 + rows written
+    uint16_t* values;
+    float* out;                 // [rows, heads, 128]
+    float* part;                // chunk partials or scores, part_bytes
+    size_t part_bytes;          // prefill_attention_part_bytes
+    long long time_stride;      // elements between consecutive positions
+    int p0, rows;               // query z is position p0 + z and attends positions 0 .. p0 + z
+    int kv_heads, groups;
+    int heads, cpb, part_chunks;   // set by launch_prefill_attention
+};
+// Workspace for batches of up to `rows` queries in a cache of `capacity` positions.
+size_t prefill_attention_part_bytes(int rows, int heads, int capacity);
+hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s);
 
 // ---- persistent layer kernel ---------------------------------------------------
 // Shapes the kernel is compiled for (head_dim 128, <= 4 query heads per kv

@@ -10,7 +10,7 @@
 //   rows<NORM | RESID_NORM>  x (+= previous down output), RMSNorm, int8 quant
 //   gemm_run                 qkv for every token (int8 MFMA, = the GEMV bits)
 //   prefill_qk_kernel        q/k head norm + RoPE, K/V rows -> fp16 cache
-//   attention (PLAIN batch)  query z attends start + z + 1 positions
+//   prompt attention         query z attends start + z + 1 positions (hq_prefill_attn.hip)
 //   rows<PLAIN>, gemm_run    o
 //   rows<RESID_NORM>, gemm   x += o, RMSNorm, gate_up
 //   rows<SWIGLU>, gemm_run   SwiGLU, down
@@ -42,7 +42,7 @@
 
 namespace hq {
 
-constexpr int kPrefillBatch = 128;      // tokens per pass over the layers
+constexpr int kPrefillBatch = 2048;     // tokens per pass over the layers
 constexpr int kPrefillMaxWidth = 10240; // intermediate size the SwiGLU row kernel holds in LDS
 
 enum RowMode { ROW_NORM = 0, ROW_RESID_NORM = 1, ROW_PLAIN = 2, ROW_SWIGLU = 3 };
@@ -245,7 +245,7 @@ __global__ void prefill_position_kernel(int32_t* position, int value) { *positio
 // Workspace layout for a model and KV capacity.
 struct PrefillLayout {
     size_t x, q8, act, qkv, qh, att, proj, gu, gemm, attn_part, total;
-    int kp, max_chunks, qkv_rows, qd;
+    int kp, qkv_rows, qd;
 };
 
 static size_t al256p(size_t v) { return (v + 255) & ~size_t(255); }
@@ -253,14 +253,13 @@ static size_t al256p(size_t v) { return (v + 255) & ~size_t(255); }
 static PrefillLayout prefill_layout(const hq_model* m, int capacity)
 {
     PrefillLayout L{};
-    const int B = kPrefillBatch;
+    const int B = std::min(kPrefillBatch, capacity);   // (no batch exceeds the cache)
     const int H = m->hidden, I = m->intermediate, D = m->head_dim;
     L.qd = m->heads * D;
     L.qkv_rows = L.qd + 2 * m->kv_heads * D;
     int kmax = H > L.qd ? H : L.qd;
     if (I > kmax) kmax = I;
     L.kp = gemm_padded_k(kmax);
-    L.max_chunks = (capacity + kAttnChunk - 1) / kAttnChunk;
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t at = off; off += al256p(bytes); return at; };
     L.x = take(size_t(B) * H * 4);
@@ -276,7 +275,7 @@ static PrefillLayout prefill_layout(const hq_model* m, int capacity)
     g = std::max<size_t>(g, gemm_scratch_bytes(B, 2 * I, H));
     g = std::max<size_t>(g, gemm_scratch_bytes(B, H, I));
     L.gemm = take(g);
-    L.attn_part = take(size_t(B) * attention_workspace_floats(m->heads, L.max_chunks, D) * 4);
+    L.attn_part = take(prefill_attention_part_bytes(B, m->heads, capacity));
     L.total = off;
     return L;
 }
@@ -619,20 +618,19 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
             qp.q = qh;
             hipLaunchKernelGGL(prefill_qk_kernel, dim3(rows, slots), dim3(kBlock), 0, s, qp);
             if (hipGetLastError() != hipSuccess) return HQ_ERR_LAUNCH;
-            AttnParams a{};
+            PrefillAttnParams a{};
             a.q = qh;
             a.keys = qp.keys;
             a.values = qp.values;
+            a.out = att;
+            a.part = reinterpret_cast<float*>(ws + L.attn_part);
+            a.part_bytes = prefill_attention_part_bytes(std::min(kPrefillBatch, st->capacity), m->heads, st->capacity);
             a.time_stride = time_stride;
-            a.context = p0 + 1;
-            a.batch = rows;
+            a.p0 = p0;
+            a.rows = rows;
             a.kv_heads = KV;
             a.groups = m->heads / KV;
-            a.head_dim = D;
-            a.max_chunks = L.max_chunks;
-            a.part = reinterpret_cast<float*>(ws + L.attn_part);
-            a.out = att;
-            if (launch_attention(a, false, s) != hipSuccess) return HQ_ERR_LAUNCH;
+            if (launch_prefill_attention(a, s) != hipSuccess) return HQ_ERR_LAUNCH;
             // o projection, residual, post-attention RMSNorm, gate_up
             rp.x = att;
             rp.add = nullptr;

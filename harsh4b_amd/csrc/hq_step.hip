@@ -172,7 +172,7 @@ static hipError_t enqueue_layers(const hq_model* m, const hq_state* st, bool emb
         a.max_chunks = Ly.max_chunks;
         a.part = reinterpret_cast<float*>(ws);
         a.out = st->attended;
-        if ((e = launch_attention(a, true, s)) != hipSuccess) return e;
+        if ((e = launch_step_attention(a, s)) != hipSuccess) return e;
 
         if ((e = layer_gemv(m, st, l, StepGemv::OResidual, s)) != hipSuccess) return e;
         if ((e = layer_gemv(m, st, l, StepGemv::GateUpSwiglu, s)) != hipSuccess) return e;

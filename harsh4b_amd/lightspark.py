@@ -325,7 +325,7 @@ class LiteSparkQwen:
         loop of forward_token over it would (the reference's prompt loop,
         cpu_lightspark.py:809-810, inference_runtime.py:177-181), with the
         same bits: every token but the last goes through hq_prefill (layer by
-        layer for up to 128 tokens at once, the projections as int8 MFMA
+        layer for up to 2048 tokens at once, the projections as int8 MFMA
         GEMMs), the last through the decode step, which computes the logits
         and the greedy token."""
         ids = np.asarray(list(token_ids), dtype=np.int64).reshape(-1)

@@ -244,7 +244,7 @@ int hq_step_layer_blocks(const hq_model* model);
 int hq_decode_step(const hq_model* model, const hq_state* state, void* stream);
 
 /* Batched prefill: consume tokens[0..count) (device int32) at positions
- * start .. start+count-1 layer by layer for up to 128 tokens at a time (the
+ * start .. start+count-1 layer by layer for up to 2048 tokens at a time (the
  * body projections as int8 MFMA GEMMs, attention batched over the tokens,
  * each query seeing its own causal context), with the arithmetic of
  * hq_decode_step, so the K/V rows written are the bits count steps would

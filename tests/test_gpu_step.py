@@ -392,3 +392,49 @@ def test_qwen3_4b_prefill_after_a_long_turn(qwen):
     earlier = [int(t) for t in rng.integers(0, 151936, 300)]
     prompt = [int(t) for t in rng.integers(0, 151936, 300)]
     _prefill_vs_steps(model, prompt, 604, start_tokens=earlier)
+
+
+@pytest.mark.parametrize("start,n", [(0, 66), (1, 15), (63, 2), (60, 150), (511, 17), (1000, 130), (0, 1050)])
+def test_qwen3_4b_prefill_attention_forms(qwen, start, n):
+    # query tiles aligned to 16 positions that begin and end inside one, on
+    # both sides of a 64-position chunk edge: single-chunk batches, chunk
+    # partials with their combine, and (1050 tokens) the stored scores
+    model, _ = qwen
+    rng = np.random.default_rng(7 * start + n)
+    a, b = model.new_state(start + n), model.new_state(start + n)
+    if start:
+        earlier = [int(t) for t in rng.integers(0, 151936, start)]
+        model.prefill(earlier, a)
+        for t in earlier:
+            model.forward_token(t, b)
+    prompt = [int(t) for t in rng.integers(0, 151936, n)]
+    la = to_host(model.prefill(prompt, a)).copy()
+    for t in prompt:
+        lb = model.forward_token(t, b)
+    assert_bits_equal(to_host(a.keys).view(np.uint16), to_host(b.keys).view(np.uint16), "keys")
+    assert_bits_equal(to_host(a.values).view(np.uint16), to_host(b.values).view(np.uint16), "values")
+    assert_bits_equal(la, to_host(lb), "logits")
+    a.check_status()
+    b.check_status()
+
+
+def test_qwen3_4b_prefill_attention_scores_computed_twice(qwen):
+    # 2000 tokens after 5000: the scores exceed the workspace, so the kernel
+    # walks the keys twice; pieces of 300 tokens keep theirs
+    model, _ = qwen
+    rng = np.random.default_rng(5)
+    gen = torch.Generator(device=dev()).manual_seed(5)
+    a, b = model.new_state(7000), model.new_state(7000)
+    for cache in ("keys", "values"):
+        hist = torch.randn((36, 5000, 8, 128), generator=gen, device=dev()).half()
+        getattr(a, cache)[:, :5000] = hist
+        getattr(b, cache)[:, :5000] = hist
+    model.stream.wait_stream(torch.cuda.current_stream())
+    a.position = b.position = 5000
+    prompt = [int(t) for t in rng.integers(0, 151936, 2000)]
+    la = to_host(model.prefill(prompt, a)).copy()
+    for i in range(0, 2000, 300):
+        lb = model.prefill(prompt[i:i + 300], b)
+    assert_bits_equal(la, to_host(lb), "logits")
+    assert_bits_equal(to_host(a.keys).view(np.uint16), to_host(b.keys).view(np.uint16), "keys")
+    assert_bits_equal(to_host(a.values).view(np.uint16), to_host(b.values).view(np.uint16), "values")
