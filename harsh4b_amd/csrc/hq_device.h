@@ -52,6 +52,28 @@ __device__ __forceinline__ float spec_expf(float x)
     return p;
 }
 
+// spec_expf without branches: the arguments outside the polynomial's range
+// are clamped into it and their results selected afterwards.
+__device__ __forceinline__ float spec_expf_sel(float x)
+{
+    const float y = fminf(fmaxf(x, -87.0f), 0x1.62e430p+6f);
+    const float n = __builtin_rintf(y * 0x1.715476p+0f);
+    float r = __builtin_fmaf(-n, 0x1.62e400p-1f, y);
+    r = __builtin_fmaf(-n, 0x1.7f7d1cp-20f, r);
+    float p = 0x1.a01a02p-13f;
+    p = __builtin_fmaf(p, r, 0x1.6c16c2p-10f);
+    p = __builtin_fmaf(p, r, 0x1.111112p-7f);
+    p = __builtin_fmaf(p, r, 0x1.555556p-5f);
+    p = __builtin_fmaf(p, r, 0x1.555556p-3f);
+    p = __builtin_fmaf(p, r, 0.5f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_fmaf(p, r, 1.0f);
+    p = __builtin_ldexpf(p, int(n));     // (exact: the result is in [2^-126, 2^128])
+    p = x < -87.0f ? 0.0f : p;
+    p = x > 0x1.62e430p+6f ? __builtin_inff() : p;
+    return x != x ? x : p;
+}
+
 // spec_expf for x <= 0 (or NaN), without branches: the exponent of e^x is
 // in [-126, 0] wherever x >= -87, so the two power-of-two multiplies are one
 // exact ldexp.

@@ -308,6 +308,7 @@ static bool launch_staged(const GemmParams& p, bool two_groups, hipStream_t s)
 static hipError_t run_gemm(const int8_t* x, const float* act, const uint8_t* w, const float* ws,
                            float* out, int m, int n, int k, int32_t* acc_out, hipStream_t s)
 {
+    if (m > kMaxBatch && gemm_tile_fits(m, n, k)) return gemm_tile_run(x, act, w, ws, out, m, n, k, acc_out, s);
     const int kp = padded_k(k);
     const int nds = (k + 127) / 128;
     const int waves = nds <= 4 * 6 ? 4 : nds <= 8 * 6 ? 8 : 16;

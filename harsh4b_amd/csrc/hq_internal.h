@@ -162,6 +162,21 @@ hipError_t gemm_run_swiglu_tail(const int8_t* x, const float* act, const uint8_t
                                 int k, const GemmTail& tail, hipStream_t s);
 hipError_t gemm_run_tail(const int8_t* x, const float* act, const uint8_t* w, const float* ws, int m, int n, int k,
                          const GemmTail& tail, hipStream_t s);
+// The GEMM for batches of more than 32 rows (hq_gemm_tile.hip), and with
+// SwiGLU in its epilogue (w: gate rows [0, n), up rows [n, 2n); out [m, n]).
+bool gemm_tile_fits(int m, int n, int k);
+hipError_t gemm_tile_run(const int8_t* x, const float* act, const uint8_t* w, const float* ws, float* out, int m,
+                         int n, int k, int32_t* acc_out, hipStream_t s);
+// The products alone, for consumers that add the sums themselves (GemmSums):
+// part[s, m, n] = 16 x the int32 sums over the s-th part of K.  Used while
+// the output has too few tiles to stream the weights (gemm_part_splits: 0
+// where it has enough); gemm_part_bytes() hold any such part.
+int gemm_part_splits(int m, int n, int k);
+size_t gemm_part_bytes();
+hipError_t gemm_tile_part(const int8_t* x, const uint8_t* w, int32_t* part, int splits, int m, int n, int k,
+                          hipStream_t s);
+hipError_t gemm_tile_swiglu(const int8_t* x, const float* act, const uint8_t* w, const float* ws, float* out, int m,
+                            int n, int k, hipStream_t s);
 hipError_t gemm_run(const int8_t* x, const float* act, const uint8_t* w, const float* ws, float* out, int m, int n,
                     int k, char* scratch, hipStream_t s);
 // The decode step's attention (q/k norms, RoPE, K/V write, attention).

@@ -8,12 +8,16 @@
 //
 // Per layer, for a batch of up to kPrefillBatch tokens:
 //   rows<NORM | RESID_NORM>  x (+= previous down output), RMSNorm, int8 quant
-//   gemm_run                 qkv for every token (int8 MFMA, = the GEMV bits)
+//   project                  qkv for every token (int8 MFMA, = the GEMV bits)
 //   prefill_qk_kernel        q/k head norm + RoPE, K/V rows -> fp16 cache
 //   prompt attention         query z attends start + z + 1 positions (hq_prefill_attn.hip)
-//   rows<PLAIN>, gemm_run    o
-//   rows<RESID_NORM>, gemm   x += o, RMSNorm, gate_up
-//   rows<SWIGLU>, gemm_run   SwiGLU, down
+//   rows<PLAIN>, project     o
+//   rows<RESID_NORM>, gemm   x += o, RMSNorm, gate_up (SwiGLU in the tiled GEMM's epilogue)
+//   rows<PLAIN | SWIGLU>, project  down
+// The last layer ends with its K/V rows.  A GEMM of up to 32 rows is
+// hq_gemm.hip's; of more, hq_gemm_tile.hip's, which while its tiles are too
+// few to stream the weights leaves two or four K parts that the next kernel
+// adds (64 tokens: 4.55 -> 3.25 ms).
 // Each row kernel restates the decode path's prologue for one token per
 // block (256-lane fmaf partials, tree sum, quantize with the spec rounding)
 // and writes the int8 row de-interleaved, as the GEMM reads it.
@@ -75,6 +79,48 @@ __global__ __launch_bounds__(kBlock) void prefill_embed_kernel(const uint8_t* em
     }
 }
 
+// A GEMM's output as its K parts (gemm_tile_part): element (m, i) is
+// (float(sum >> 4) * act[m]) * ws[i], the GEMM epilogue's operations.
+struct GemmSums {
+public:
+    const int32_t* part;    // nullable: [splits, rows, n]
+    int splits, rows, n;
+    const float* act;       // [rows]
+    const float* ws;        // [n]
+
+    // elements (m, i0 + step * j) of row m, zero from i = end on; every load
+    // goes out before the first sum (two or four parts: gemm_part_splits)
+    template <int N>
+    __device__ __forceinline__ void row(int m, int i0, int step, int end, float (&v)[N]) const
+    {
+        if (splits == 2) row_parts<2>(m, i0, step, end, v);
+        else row_parts<4>(m, i0, step, end, v);
+    }
+
+private:
+    template <int S, int N>
+    __device__ __forceinline__ void row_parts(int m, int i0, int step, int end, float (&v)[N]) const
+    {
+        const float act_m = act[m];
+        int32_t q[N][S];
+        float w[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int i = min(i0 + step * j, end - 1);
+            w[j] = ws[i];
+#pragma unroll
+            for (int s = 0; s < S; ++s) q[j][s] = part[(size_t(s) * rows + m) * n + i];
+        }
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            int32_t sum = q[j][0];
+#pragma unroll
+            for (int s = 1; s < S; ++s) sum += q[j][s];
+            v[j] = i0 + step * j < end ? (float(sum >> 4) * act_m) * w[j] : 0.0f;
+        }
+    }
+};
+
 struct RowParams {
     float* x;               // [batch, k] (NORM, RESID_NORM: the residual stream; PLAIN: the input rows)
     const float* add;       // RESID_NORM: [batch, k] added to x first (x is updated)
@@ -84,6 +130,7 @@ struct RowParams {
     int k, kp;              // width; row stride of q (gemm_padded_k(k))
     int8_t* q;              // [*, kp] de-interleaved
     float* act;             // [batch]
+    GemmSums sums;          // with parts: in place of add (RESID_NORM, n = k) or gate_up (SWIGLU, n = 2k)
 };
 
 // One token (block) per row: the prologue of the step's GEMVs.  Thread t
@@ -107,6 +154,7 @@ __global__ __launch_bounds__(THREADS) void prefill_rows_kernel(RowParams p)
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int k = p.k;
+    const bool parts = p.sums.part != nullptr;
     float v[NPT];
     if constexpr (MODE == ROW_SWIGLU) {
         const float* g = p.gate_up + size_t(m) * 2 * k;
@@ -114,8 +162,12 @@ __global__ __launch_bounds__(THREADS) void prefill_rows_kernel(RowParams p)
 #pragma unroll
         for (int j = 0; j < NPT; ++j) {
             const int i = tid + THREADS * j;
-            gv[j] = i < k ? g[i] : 0.0f;
-            uv[j] = i < k ? g[k + i] : 0.0f;
+            gv[j] = i < k && !parts ? g[i] : 0.0f;
+            uv[j] = i < k && !parts ? g[k + i] : 0.0f;
+        }
+        if (parts) {
+            p.sums.row(m, tid, THREADS, k, gv);
+            p.sums.row(m, k + tid, THREADS, 2 * k, uv);
         }
 #pragma unroll
         for (int j = 0; j < NPT; ++j) {
@@ -133,11 +185,21 @@ __global__ __launch_bounds__(THREADS) void prefill_rows_kernel(RowParams p)
         }
         float sum[MODE == ROW_RESID_NORM ? NPT : 1];
         if constexpr (MODE == ROW_RESID_NORM) {
-            const float* ar = p.add + size_t(m) * k;
+            float add[NPT];
+            if (parts) {
+                p.sums.row(m, tid, THREADS, k, add);
+            } else {
+                const float* ar = p.add + size_t(m) * k;
+#pragma unroll
+                for (int j = 0; j < NPT; ++j) {
+                    const int i = tid + THREADS * j;
+                    add[j] = i < k ? ar[i] : 0.0f;
+                }
+            }
 #pragma unroll
             for (int j = 0; j < NPT; ++j) {
                 const int i = tid + THREADS * j;
-                v[j] = i < k ? v[j] + ar[i] : 0.0f;
+                v[j] = i < k ? v[j] + add[j] : 0.0f;
                 sum[j] = v[j];
             }
         }
@@ -193,6 +255,7 @@ struct QkParams {
     uint16_t* keys;         // this layer's cache
     uint16_t* values;
     float* q;               // [batch, heads * D]
+    GemmSums sums;          // with parts: in place of qkv
 };
 
 // Wave w of block (m, b) handles head slot 4b + w of token m: query heads
@@ -209,8 +272,17 @@ __global__ __launch_bounds__(kBlock) void prefill_qk_kernel(QkParams p)
     const int total = p.heads + 2 * p.kv_heads;
     if (slot >= total) return;
     const int pos = p.start + m;
-    const float* src = p.qkv + size_t(m) * total * D + size_t(slot) * D;
-    const float x0 = src[lane], x1 = src[lane + 64];
+    float x0, x1;
+    if (p.sums.part) {
+        float x[2];
+        p.sums.row(m, slot * D + lane, 64, total * D, x);
+        x0 = x[0];
+        x1 = x[1];
+    } else {
+        const float* src = p.qkv + size_t(m) * total * D + size_t(slot) * D;
+        x0 = src[lane];
+        x1 = src[lane + 64];
+    }
     if (slot >= p.heads + p.kv_heads) {
         uint16_t* vdst = p.values + size_t(pos) * p.time_stride + size_t(slot - p.heads - p.kv_heads) * D;
         vdst[lane] = f32_to_f16(x0);
@@ -244,7 +316,7 @@ __global__ void prefill_position_kernel(int32_t* position, int value) { *positio
 
 // Workspace layout for a model and KV capacity.
 struct PrefillLayout {
-    size_t x, q8, act, qkv, qh, att, proj, gu, gemm, attn_part, total;
+    size_t x, q8, act, qkv, qh, att, proj, gu, gemm, part, attn_part, total;
     int kp, qkv_rows, qd;
 };
 
@@ -275,6 +347,7 @@ static PrefillLayout prefill_layout(const hq_model* m, int capacity)
     g = std::max<size_t>(g, gemm_scratch_bytes(B, 2 * I, H));
     g = std::max<size_t>(g, gemm_scratch_bytes(B, H, I));
     L.gemm = take(g);
+    L.part = take(gemm_part_bytes());
     L.attn_part = take(prefill_attention_part_bytes(B, m->heads, capacity));
     L.total = off;
     return L;
@@ -298,21 +371,22 @@ static bool batch_fits(const hq_model* m) { return prefill_fits(m) && m->heads <
 template <int MODE>
 static void launch_rows(const RowParams& p, int rows, hipStream_t s)
 {
-    if constexpr (MODE != ROW_SWIGLU) {
+    if constexpr (MODE == ROW_SWIGLU || MODE == ROW_PLAIN) {
+        // 16 waves share the row's exp / divide work (its maximum is
+        // order-free); 9.6 -> 6.0 us for 8 SwiGLU rows of 9728 against 256
+        // threads
+        constexpr int T = 4 * kBlock;
+        if (p.k <= T * 4)
+            hipLaunchKernelGGL((prefill_rows_kernel<MODE, 4, T>), dim3(rows), dim3(T), 0, s, p);
+        else
+            hipLaunchKernelGGL((prefill_rows_kernel<MODE, 10, T>), dim3(rows), dim3(T), 0, s, p);
+    } else {
         if (p.k <= kBlock * 10)
             hipLaunchKernelGGL((prefill_rows_kernel<MODE, 10, kBlock>), dim3(rows), dim3(kBlock), 0, s, p);
         else if (p.k <= kBlock * 16)
             hipLaunchKernelGGL((prefill_rows_kernel<MODE, 16, kBlock>), dim3(rows), dim3(kBlock), 0, s, p);
         else
             hipLaunchKernelGGL((prefill_rows_kernel<MODE, 40, kBlock>), dim3(rows), dim3(kBlock), 0, s, p);
-    } else {
-        // SwiGLU: 16 waves share the row's exp / divide work (its maximum
-        // is order-free); 9.6 -> 6.0 us for 8 rows of 9728 against 256 threads
-        constexpr int T = 4 * kBlock;
-        if (p.k <= T * 4)
-            hipLaunchKernelGGL((prefill_rows_kernel<MODE, 4, T>), dim3(rows), dim3(T), 0, s, p);
-        else
-            hipLaunchKernelGGL((prefill_rows_kernel<MODE, 10, T>), dim3(rows), dim3(T), 0, s, p);
     }
 }
 
@@ -587,6 +661,22 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
         hipLaunchKernelGGL(prefill_embed_kernel, dim3(rows), dim3(kBlock), 0, s, m->embedding, m->embedding_scales,
                            m->vocab, H, tokens + b0, st->status, x);
         if (hipGetLastError() != hipSuccess) return HQ_ERR_LAUNCH;
+        // A GEMM whose consumer is one of this file's kernels: as K parts the
+        // consumer adds (few rows), else into `out`.
+        int32_t* part = reinterpret_cast<int32_t*>(ws + L.part);
+        auto project = [&](const uint8_t* w, const float* scales, float* out, int n, int k, GemmSums& sums) {
+            sums = GemmSums{};
+            const int splits = rows > 32 ? gemm_part_splits(rows, n, k) : 0;
+            if (splits == 0) return gemm_run(q8, act, w, scales, out, rows, n, k, gemm, s);
+            sums.part = part;
+            sums.splits = splits;
+            sums.rows = rows;
+            sums.n = n;
+            sums.act = act;
+            sums.ws = scales;
+            return gemm_tile_part(q8, w, part, splits, rows, n, k, s);
+        };
+        GemmSums down{};
         for (int l = 0; l < m->layers; ++l) {
             const hq_layer& Ly = m->layer[l];
             RowParams rp{};
@@ -596,13 +686,13 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
             // input RMSNorm (adding the previous layer's down output first)
             rp.x = x;
             rp.add = proj;
+            rp.sums = down;
             rp.gamma = Ly.input_norm;
             rp.k = H;
             int e = run_rows(l == 0 ? ROW_NORM : ROW_RESID_NORM, rp, rows, s);
             if (e) return e;
-            if (gemm_run(q8, act, Ly.qkv, Ly.qkv_scales, qkv, rows, L.qkv_rows, H, gemm, s) != hipSuccess)
-                return HQ_ERR_LAUNCH;
             QkParams qp{};
+            if (project(Ly.qkv, Ly.qkv_scales, qkv, L.qkv_rows, H, qp.sums) != hipSuccess) return HQ_ERR_LAUNCH;
             qp.qkv = qkv;
             qp.q_norm = Ly.q_norm;
             qp.k_norm = Ly.k_norm;
@@ -618,6 +708,7 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
             qp.q = qh;
             hipLaunchKernelGGL(prefill_qk_kernel, dim3(rows, slots), dim3(kBlock), 0, s, qp);
             if (hipGetLastError() != hipSuccess) return HQ_ERR_LAUNCH;
+            if (l == m->layers - 1) break;   // its K/V rows are written: nothing reads the rest
             PrefillAttnParams a{};
             a.q = qh;
             a.keys = qp.keys;
@@ -634,27 +725,30 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
             // o projection, residual, post-attention RMSNorm, gate_up
             rp.x = att;
             rp.add = nullptr;
+            rp.sums = GemmSums{};
             rp.gamma = nullptr;
             rp.k = m->heads * D;
             if ((e = run_rows(ROW_PLAIN, rp, rows, s))) return e;
-            if (gemm_run(q8, act, Ly.o, Ly.o_scales, proj, rows, H, rp.k, gemm, s) != hipSuccess) return HQ_ERR_LAUNCH;
+            if (project(Ly.o, Ly.o_scales, proj, H, rp.k, rp.sums) != hipSuccess) return HQ_ERR_LAUNCH;
             rp.x = x;
             rp.add = proj;
             rp.gamma = Ly.post_norm;
             rp.k = H;
             if ((e = run_rows(ROW_RESID_NORM, rp, rows, s))) return e;
-            if (gemm_run(q8, act, Ly.gate_up, Ly.gate_up_scales, gu, rows, 2 * I, H, gemm, s) != hipSuccess)
-                return HQ_ERR_LAUNCH;
-            // SwiGLU, down (its residual is added at the next layer's input;
-            // the last layer's is not needed: no logits for these tokens)
-            rp.x = nullptr;
+            // SwiGLU (in the tiled GEMM's epilogue where it writes whole
+            // sums), down (its residual is added at the next layer's input)
+            const bool fused = rows > 32 && gemm_part_splits(rows, 2 * I, H) == 0 && gemm_tile_fits(rows, 2 * I, H);
+            rp.sums = GemmSums{};
+            const hipError_t ge = fused ? gemm_tile_swiglu(q8, act, Ly.gate_up, Ly.gate_up_scales, gu, rows, I, H, s)
+                                        : project(Ly.gate_up, Ly.gate_up_scales, gu, 2 * I, H, rp.sums);
+            if (ge != hipSuccess) return HQ_ERR_LAUNCH;
+            rp.x = gu;
             rp.add = nullptr;
             rp.gate_up = gu;
             rp.gamma = nullptr;
             rp.k = I;
-            if ((e = run_rows(ROW_SWIGLU, rp, rows, s))) return e;
-            if (gemm_run(q8, act, Ly.down, Ly.down_scales, proj, rows, H, I, gemm, s) != hipSuccess)
-                return HQ_ERR_LAUNCH;
+            if ((e = run_rows(fused ? ROW_PLAIN : ROW_SWIGLU, rp, rows, s))) return e;
+            if (project(Ly.down, Ly.down_scales, proj, H, I, down) != hipSuccess) return HQ_ERR_LAUNCH;
         }
     }
     hipLaunchKernelGGL(prefill_position_kernel, dim3(1), dim3(1), 0, s, st->position, start + count);

@@ -391,3 +391,22 @@ def test_batched_gemm_wide_rows(m):
     assert_bits_equal(to_host(acc), oracle.int4_i8_gemm_acc(q, packed, rows, width), "wide acc")
     ref = np.stack([oracle.int4_i8_gemv(q[i], packed, s, a[i], rows, width) for i in range(m)])
     assert_bits_equal(to_host(out), ref, "wide out")
+
+
+@pytest.mark.parametrize("m,rows,width", [(33, 67, 160), (64, 64, 128), (65, 63, 352), (200, 1000, 1056),
+                                          (640, 1400, 160), (641, 1409, 256), (1030, 4000, 96), (1024, 4097, 224)])
+def test_batched_gemm_tiles(m, rows, width):
+    # more than 32 rows: 64 x 64, 64 x 128 and 128 x 128 output tiles with
+    # ragged last tiles, K below, at and between whole 128-column steps
+    ls = lightspark()
+    rng = np.random.default_rng(m + rows + width)
+    packed = oracle.pack_int4(random_int4(rng, rows, width))
+    s = rng.uniform(0.005, 0.02, rows).astype(np.float32)
+    q = rng.integers(-127, 128, (m, width)).astype(np.int8)
+    a = rng.uniform(0.001, 0.01, m).astype(np.float32)
+    p = ls.LiteSparkProjection(to_dev(packed), to_dev(s))
+    acc = torch.empty((m, rows), dtype=torch.int32, device=dev())
+    out = ls.int4_i8_gemm(to_dev(q), to_dev(a), p, acc_out=acc)
+    ref = oracle.int4_i8_gemm_acc(q, packed, rows, width)
+    assert_bits_equal(to_host(acc), ref, "acc")
+    assert_bits_equal(to_host(out), (ref.astype(np.float32) * a[:, None]) * s[None, :], "out")

@@ -438,3 +438,16 @@ def test_qwen3_4b_prefill_attention_scores_computed_twice(qwen):
     assert_bits_equal(la, to_host(lb), "logits")
     assert_bits_equal(to_host(a.keys).view(np.uint16), to_host(b.keys).view(np.uint16), "keys")
     assert_bits_equal(to_host(a.values).view(np.uint16), to_host(b.values).view(np.uint16), "values")
+
+
+@pytest.mark.parametrize("n", [33, 65, 130, 700])
+def test_ragged_model_prefill_matches_token_steps(n):
+    # widths that are no multiple of 128 columns, a row count of no tile:
+    # the GEMMs in K parts, whole, and with SwiGLU in the epilogue
+    from harsh4b_amd.synthetic import random_model
+    config = {"hidden_size": 352, "intermediate_size": 3232, "num_attention_heads": 6, "num_key_value_heads": 2,
+              "head_dim": 128, "num_hidden_layers": 3, "vocab_size": 515, "rms_norm_eps": 1e-6,
+              "rope_theta": 1000000, "max_position_embeddings": 1024}
+    model = random_model(config, 3, dev())
+    rng = np.random.default_rng(n)
+    _prefill_vs_steps(model, [int(t) for t in rng.integers(0, 515, n)], n + 8, start_tokens=[5, 6])
