@@ -69,9 +69,9 @@ int hq_quantize_activation(const float* x, int n, int8_t* q, float* act_scale, v
 int hq_rmsnorm(const float* x, const float* gamma, float* y, int n, float eps, void* stream);
 
 /* ------------------------------------------- GQA decode attention --
- * Fused single-token GQA attention: score, softmax and V accumulation in
- * one launch (per 64-position chunk, with the chunks' combine in the same
- * launch).  Replaces litespark_gqa_decode (cpu_kernels/
+ * Fused single-token GQA attention: score, softmax and V accumulation per
+ * 64-position chunk, with the chunks' combine in the same launch or, for long
+ * contexts, a second one.  Replaces litespark_gqa_decode (cpu_kernels/
  * litespark_int4.cpp:160-171, bound at cpu_lightspark.py:102-111) with the
  * same argument list and meaning:
  * query fp32 [kv_heads*groups, head_dim], heads ordered [kv_head, group];

@@ -410,3 +410,22 @@ def test_batched_gemm_tiles(m, rows, width):
     ref = oracle.int4_i8_gemm_acc(q, packed, rows, width)
     assert_bits_equal(to_host(acc), ref, "acc")
     assert_bits_equal(to_host(out), (ref.astype(np.float32) * a[:, None]) * s[None, :], "out")
+
+
+@pytest.mark.parametrize("kv,g,d,ctx", [(2, 1, 16, 4097), (1, 8, 32, 8257), (2, 5, 64, 8193), (2, 4, 128, 33000),
+                                        (1, 7, 128, 33089)])
+def test_gqa_long_contexts(kv, g, d, ctx):
+    # past one combine batch (two, with more than four query heads): the items
+    # and combine launches, one and two rounds of the combine, ragged last
+    # chunks; the workspace is left at zero for a short call
+    ls = lightspark()
+    rng = np.random.default_rng(ctx + d)
+    q = rng.standard_normal((kv * g, d)).astype(np.float32)
+    k = rng.standard_normal((ctx, kv, d)).astype(np.float16)
+    v = rng.standard_normal((ctx, kv, d)).astype(np.float16)
+    qd, kd, vd = to_dev(q), to_dev(k), to_dev(v)
+    out = torch.empty((kv * g, d), dtype=torch.float32, device=dev())
+    for n in (ctx, 100, ctx - 1, 4096):
+        ls.gqa_decode(qd, kd, vd, out, n, kv, g, d)
+        ref = oracle.gqa_decode_split(q, k[:n].view(np.uint16), v[:n].view(np.uint16), n, kv, g, d)
+        assert_bits_equal(to_host(out), np.asarray(ref).reshape(kv * g, d), f"context {n}")
