@@ -22,6 +22,7 @@ an error.
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import numpy as np
@@ -56,9 +57,11 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 
 def _stream_handle(stream: torch.cuda.Stream | None) -> int | None:
     """The HIP stream of `stream`, or torch's current stream when None (so
-    the op is ordered with the caller's other torch work)."""
+    the op is ordered with the caller's other torch work).  The raw handle,
+    without a Stream object: an op's host time is the whole of a small GEMV's
+    call."""
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return stream.cuda_stream
 
 
@@ -605,7 +608,8 @@ def _zeroed_workspace(kind: tuple, nbytes: int, device, stream=None) -> torch.Te
     and overlapping calls on one workspace would share its ticket counters.
     The zero fill runs on the current stream; a given `stream` is made to
     wait for it."""
-    handle = (stream if stream is not None else torch.cuda.current_stream(device)).cuda_stream
+    handle = (stream.cuda_stream if stream is not None
+              else torch._C._cuda_getCurrentRawStream(torch.cuda._utils._get_device_index(device)))
     key = (*kind, handle)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
@@ -661,6 +665,11 @@ def rmsnorm(x: torch.Tensor, gamma: torch.Tensor, eps: float, out: torch.Tensor 
     return out
 
 
+@functools.lru_cache(maxsize=1024)
+def _gqa_workspace_bytes(capacity: int, kv_heads: int, groups: int, head_dim: int) -> int:
+    return _native.lib().hq_gqa_workspace_bytes(capacity, kv_heads, groups, head_dim)
+
+
 def gqa_decode(query: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, out: torch.Tensor,
                context: int, kv_heads: int, groups: int, head_dim: int, stream=None) -> torch.Tensor:
     """Fused GQA decode over an fp16 [capacity, kv_heads, head_dim] cache
@@ -669,19 +678,25 @@ def gqa_decode(query: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, ou
     if keys.dtype != torch.float16 or values.dtype != torch.float16:
         raise ValueError("keys/values must be float16")
     shape = (keys.shape[0], kv_heads, head_dim)
-    if (keys.dim() != 3 or tuple(keys.shape) != shape or tuple(values.shape) != shape
+    if (keys.dim() != 3 or keys.shape != shape or values.shape != shape
             or not keys.is_contiguous() or not values.is_contiguous()):
         raise ValueError("keys/values must be contiguous float16 [capacity, kv_heads, head_dim]")
     capacity = int(keys.shape[0])
     if context < 1 or context > capacity:
         raise ValueError("context outside the cache")
     lib = _native.lib()
-    nbytes = lib.hq_gqa_workspace_bytes(capacity, kv_heads, groups, head_dim)
-    ws = _zeroed_workspace(("gqa", query.device.index), nbytes, query.device, stream)
+    nbytes = _gqa_workspace_bytes(capacity, kv_heads, groups, head_dim)
+    device = query.device
+    ws = _zeroed_workspace(("gqa", device.index), nbytes, device, stream)
     check(lib.hq_gqa_decode(query.data_ptr(), keys.data_ptr(), values.data_ptr(), ws.data_ptr(),
                             out.data_ptr(), context, kv_heads, groups, head_dim,
                             capacity, _stream_handle(stream)), "hq_gqa_decode")
     return out
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_workspace_bytes(m: int, rows: int, width: int) -> int:
+    return _native.lib().hq_gemm_workspace_bytes(m, rows, width)
 
 
 def int4_i8_gemm(x_q: torch.Tensor, act_scales: torch.Tensor, projection: LiteSparkProjection,
@@ -692,12 +707,12 @@ def int4_i8_gemm(x_q: torch.Tensor, act_scales: torch.Tensor, projection: LiteSp
     if out is None:
         out = torch.empty((m, projection.output_size), dtype=torch.float32, device=x_q.device)
     lib = _native.lib()
-    nbytes = lib.hq_gemm_workspace_bytes(m, projection.output_size, projection.input_size)
-    ws = _zeroed_workspace(("gemm", x_q.device.index, m, projection.output_size,
-                            projection.input_size), nbytes, x_q.device, stream)
+    rows, width = projection.output_size, projection.input_size
+    ws = _zeroed_workspace(("gemm", x_q.device.index, m, rows, width), _gemm_workspace_bytes(m, rows, width),
+                           x_q.device, stream)
     check(lib.hq_int4_i8_gemm(x_q.data_ptr(), act_scales.data_ptr(), projection.weights.data_ptr(),
-                              projection.scales.data_ptr(), out.data_ptr(), m, projection.output_size,
-                              projection.input_size, _ptr(acc_out), ws.data_ptr(),
+                              projection.scales.data_ptr(), out.data_ptr(), m, rows, width,
+                              _ptr(acc_out), ws.data_ptr(),
                               _stream_handle(stream)), "hq_int4_i8_gemm")
     return out
 
@@ -709,12 +724,11 @@ def quant_int4_gemm(x: torch.Tensor, projection: LiteSparkProjection, out: torch
     if out is None:
         out = torch.empty((m, projection.output_size), dtype=torch.float32, device=x.device)
     lib = _native.lib()
-    nbytes = lib.hq_gemm_workspace_bytes(m, projection.output_size, projection.input_size)
-    ws = _zeroed_workspace(("gemm", x.device.index, m, projection.output_size,
-                            projection.input_size), nbytes, x.device, stream)
+    rows, width = projection.output_size, projection.input_size
+    ws = _zeroed_workspace(("gemm", x.device.index, m, rows, width), _gemm_workspace_bytes(m, rows, width),
+                           x.device, stream)
     check(lib.hq_quant_int4_gemm(x.data_ptr(), projection.weights.data_ptr(), projection.scales.data_ptr(),
-                                 out.data_ptr(), m, projection.output_size, projection.input_size,
-                                 _ptr(q_out), _ptr(act_out), _ptr(acc_out), ws.data_ptr(),
+                                 out.data_ptr(), m, rows, width, _ptr(q_out), _ptr(act_out), _ptr(acc_out), ws.data_ptr(),
                                  _stream_handle(stream)), "hq_quant_int4_gemm")
     return out
 
@@ -768,15 +782,18 @@ def sample_token(logits: torch.Tensor, generated, repetition_penalty: float, tem
     k = min(int(top_k), n)
     lib = _native.lib()
     ws = _zeroed_workspace(("sample", device.index), lib.hq_sample_workspace_bytes(n, k), device, stream)
-    gen = torch.from_numpy(ids).to(device) if ids.size else None
-    draw = torch.tensor([float(u)], dtype=torch.float64, device=device)
-    out = torch.empty(1, dtype=torch.int32, device=device)
-    ranked = torch.empty(k, dtype=torch.int32, device=device)
-    probs = torch.empty(k, dtype=torch.float32, device=device)
-    check(lib.hq_sample_token(logits.data_ptr(), n, _ptr(gen), int(ids.size), float(repetition_penalty),
-                              float(temperature), int(top_k), float(top_p), draw.data_ptr(), out.data_ptr(),
-                              ranked.data_ptr(), probs.data_ptr(), ws.data_ptr(), _stream_handle(stream)),
-          "hq_sample_token")
+    # one copy each way: the draw and the ids in, the token, the ranked ids
+    # and their probabilities out (five copies were most of a call's time)
+    staged = np.empty(8 + 4 * ids.size, dtype=np.uint8)
+    staged[:8].view(np.float64)[0] = float(u)
+    staged[8:].view(np.int32)[:] = ids
+    draw = torch.from_numpy(staged).to(device)
+    out = torch.empty(1 + 2 * k, dtype=torch.int32, device=device)
+    check(lib.hq_sample_token(logits.data_ptr(), n, draw.data_ptr() + 8 if ids.size else None, int(ids.size),
+                              float(repetition_penalty), float(temperature), int(top_k), float(top_p),
+                              draw.data_ptr(), out.data_ptr(), out.data_ptr() + 4, out.data_ptr() + 4 + 4 * k,
+                              ws.data_ptr(), _stream_handle(stream)), "hq_sample_token")
     if stream is not None:
         stream.synchronize()
-    return int(out.item()), ranked.cpu().numpy(), probs.cpu().numpy()
+    host = out.cpu().numpy()
+    return int(host[0]), host[1:1 + k], host[1 + k:].view(np.float32)
