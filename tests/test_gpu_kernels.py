@@ -429,3 +429,17 @@ def test_gqa_long_contexts(kv, g, d, ctx):
         ls.gqa_decode(qd, kd, vd, out, n, kv, g, d)
         ref = oracle.gqa_decode_split(q, k[:n].view(np.uint16), v[:n].view(np.uint16), n, kv, g, d)
         assert_bits_equal(to_host(out), np.asarray(ref).reshape(kv * g, d), f"context {n}")
+
+
+@pytest.mark.parametrize("n,top_k", [(151936, 65), (151936, 256), (151936, 257), (9000, 1365), (20481, 1366),
+                                     (12289, 2048), (8192, 129), (300, 300), (130, 2048)])
+@pytest.mark.parametrize("flat", [False, True])
+def test_sampler_merge_tree_and_sums(n, top_k, flat):
+    # one wave or the block for the draw, rank and bitonic sorts, merge nodes of
+    # two and three lists with lone children, pairwise sums of one and more
+    # leaves; flat: every probability alike, so top-p cuts in the middle
+    rng = np.random.default_rng(n * 7 + top_k)
+    logits = (rng.standard_normal(n) * (1e-3 if flat else 3.0)).astype(np.float32)
+    logits[rng.integers(0, n, 5)] = -np.inf
+    for u, top_p in ((0.0, 1.0), (0.37, 1e-6), (float(rng.random()), 0.5), (0.9999999, 0.95)):
+        check_sample(logits, [1, n // 2], 1.2, 0.9, top_k, top_p, u, f"n={n} k={top_k} u={u} p={top_p} flat={flat}")
