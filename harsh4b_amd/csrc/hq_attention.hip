@@ -1044,14 +1044,11 @@ __global__ __launch_bounds__(kBlock) void attention_combine_kernel(AttnParams a)
         const int pos = *a.position;
         if (pos < 0 || pos >= a.capacity) return;   // (flagged by attention_kernel)
         n = pos + 1;
-    } else if (a.table) {
-        const int zpos = *a.table->position[z];
-        n = min(max(zpos, 0), a.table->capacity[z] - 1) + 1;
     } else {
         n = a.context + z;
     }
     const int nc = (n + C - 1) / C;
-    if (nc <= 1) return;                       // attention_kernel combined it in-block
+    if (nc <= 1) return;                       // (its chunk's block wrote the output)
     const int heads = a.kv_heads * a.groups;
     const int tid = threadIdx.x;
     const int hl = tid / D, d = tid % D;

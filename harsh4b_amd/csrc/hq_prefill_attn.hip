@@ -27,7 +27,7 @@
 // Bound by fp32 arithmetic: the fp32 matrix instructions (256 of 32 cycles per
 // 16 queries, 64 keys and head) and the fp32 vector instructions (about 800
 // of 4 cycles: conversions, tree sums, exponentials) do not run side by side.
-// 2000 tokens of 32 heads: 438 us a layer (1890 us with one query per block
+// 2000 tokens of 32 heads: 440 us a layer (1890 us with one query per block
 // on the vector unit, 672 us with the scores computed twice), 75 TFLOP/s.
 #include <algorithm>
 
@@ -41,6 +41,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kPaTile = 16;      // queries per wave
 constexpr int kPaWaves = 4;      // waves (query tile, head) per block, one kv head
 constexpr int kPaD = 128;
+constexpr int kPaCUs = 256;      // (for the order of the blocks only)
 
 template <int GROUP>
 __device__ __forceinline__ f32x16 mfma1(float a, float b, f32x16 c)
@@ -247,7 +248,9 @@ __device__ __forceinline__ void pa_combine(float M, float m, float l, const f32x
 
 // A wave's place in the launch: block b serves kv head b % kv_heads and four
 // (query tile, head) slots of it, the blocks with the longest contexts
-// first.  Everything but pos, z and store is wave-uniform.
+// first -- but the second block of each CU in the opposite order, so that the
+// blocks a CU starts with sum to about the same work (2000 tokens: 72 to 48
+// chunks per wave slot otherwise, 64 to 56 so).  Everything but pos, z and store is wave-uniform.
 struct PaPlace {
     int kvh, h, tile, nc, nc_block;   // tile: 16 positions from 16 * tile; nc: its chunks
     int slot;
@@ -260,7 +263,11 @@ struct PaPlace {
         kvh = blockIdx.x % p.kv_heads;
         const int tile0 = p.p0 / kPaTile;
         const int slots = ((p.p0 + p.rows - 1) / kPaTile - tile0 + 1) * p.groups;
-        const int slot0 = ((slots + kPaWaves - 1) / kPaWaves - 1 - int(blockIdx.x) / p.kv_heads) * kPaWaves;
+        const int groups = (slots + kPaWaves - 1) / kPaWaves;   // blocks per kv head
+        int rank = int(blockIdx.x) / p.kv_heads;
+        const int round = kPaCUs / p.kv_heads;
+        if (rank >= round && rank < 2 * round && 2 * round <= groups) rank = 3 * round - 1 - rank;
+        const int slot0 = (groups - 1 - rank) * kPaWaves;
         slot = min(slot0 + wave, slots - 1);
         live = slot0 + wave < slots;
         tile = tile0 + slot / p.groups;
