@@ -33,15 +33,14 @@
 
 #include "hq_device.h"
 #include "hq_internal.h"
+#include "hq_prefill_place.h"
 
 namespace hq {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kPaTile = 16;      // queries per wave
-constexpr int kPaWaves = 4;      // waves (query tile, head) per block, one kv head
 constexpr int kPaD = 128;
-constexpr int kPaCUs = 256;      // (for the order of the blocks only)
+static_assert(kPaChunk == kAttnChunk, "the placement counts the spec's chunks");
 
 template <int GROUP>
 __device__ __forceinline__ f32x16 mfma1(float a, float b, f32x16 c)
@@ -246,39 +245,23 @@ __device__ __forceinline__ void pa_combine(float M, float m, float l, const f32x
     }
 }
 
-// A wave's place in the launch: block b serves kv head b % kv_heads and four
-// (query tile, head) slots of it, the blocks with the longest contexts
-// first -- but the second block of each CU in the opposite order, so that the
-// blocks a CU starts with sum to about the same work (2000 tokens: 72 to 48
-// chunks per wave slot otherwise, 64 to 56 so).  Everything but pos, z and store is wave-uniform.
-struct PaPlace {
-    int kvh, h, tile, nc, nc_block;   // tile: 16 positions from 16 * tile; nc: its chunks
-    int slot;
+__host__ __device__ constexpr PaBatch pa_batch(const PrefillAttnParams& p)
+{
+    return PaBatch{p.p0, p.rows, p.kv_heads, p.groups};
+}
+
+// A wave's slot (wave-uniform), and this lane's query in it.
+struct PaPlace : PaSlot {
     int pos, z;                       // this lane's query position and row (clamped into the batch)
-    bool live, store;
+    bool store;
 
     __device__ __forceinline__ explicit PaPlace(const PrefillAttnParams& p)
+        : PaSlot(pa_slot(pa_batch(p), int(blockIdx.x), __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave)))
     {
-        const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kWave);
-        kvh = blockIdx.x % p.kv_heads;
-        const int tile0 = p.p0 / kPaTile;
-        const int slots = ((p.p0 + p.rows - 1) / kPaTile - tile0 + 1) * p.groups;
-        const int groups = (slots + kPaWaves - 1) / kPaWaves;   // blocks per kv head
-        int rank = int(blockIdx.x) / p.kv_heads;
-        const int round = kPaCUs / p.kv_heads;
-        if (rank >= round && rank < 2 * round && 2 * round <= groups) rank = 3 * round - 1 - rank;
-        const int slot0 = (groups - 1 - rank) * kPaWaves;
-        slot = min(slot0 + wave, slots - 1);
-        live = slot0 + wave < slots;
-        tile = tile0 + slot / p.groups;
-        h = kvh * p.groups + slot % p.groups;
-        nc = chunks(tile);
-        nc_block = chunks(tile0 + min(slot0 + kPaWaves - 1, slots - 1) / p.groups);
         pos = tile * kPaTile + int(threadIdx.x & 15);
         z = min(max(pos - p.p0, 0), p.rows - 1);
         store = live && pos >= p.p0 && pos < p.p0 + p.rows;
     }
-    static __device__ __forceinline__ int chunks(int tile) { return tile * kPaTile / kAttnChunk + 1; }
     // 16-key blocks of chunk c that every query of the tile sees whole
     __device__ __forceinline__ int full(int c) const { return min(4, tile - c * (kAttnChunk / kPaTile)); }
 };
@@ -467,7 +450,7 @@ __global__ __launch_bounds__(kPaWaves * kWave, 2) void prefill_attention_walk_ke
         if (PART) M = m;                                 // one chunk
         pa_combine(M, m, l, ae, ao, L, oe, oo);
     }
-    if (w.store && !(PART && w.nc > 1)) pa_store_out(p, w, L, oe, oo);
+    if (w.store && pa_stores_output(PART, w.nc, c_begin)) pa_store_out(p, w, L, oe, oo);
 }
 
 // Workspace limit (larger batches or contexts take the two-pass form, which
@@ -498,9 +481,7 @@ hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s)
     if (a.rows < 1 || a.p0 < 0 || a.groups < 1 || a.groups > 8) return hipErrorInvalidValue;
     PrefillAttnParams p = a;
     p.heads = a.kv_heads * a.groups;
-    const int tile0 = p.p0 / kPaTile;
-    const int tiles = (p.p0 + p.rows - 1) / kPaTile - tile0 + 1;
-    const int blocks = (tiles * p.groups + kPaWaves - 1) / kPaWaves * p.kv_heads;
+    const int blocks = pa_blocks_per_kv(pa_batch(p)) * p.kv_heads;
     const int nc = (p.p0 + p.rows - 1) / kAttnChunk + 1;
     AttnParams c{};
     c.q = p.q;
@@ -521,11 +502,11 @@ hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s)
     // fewer blocks than CUs: chunk partials from several blocks per tile, as
     // many as fill two blocks per CU
     if (blocks < 256 && pa_part_bytes(p.rows, p.heads, nc) <= p.part_bytes) {
-        const int splits = std::min(nc, std::max(1, 512 / blocks));
-        p.cpb = (nc + splits - 1) / splits;
+        const PaPartGrid g = pa_part_grid(pa_batch(p));
+        p.cpb = g.cpb;
         p.part_chunks = nc;
-        hipLaunchKernelGGL(prefill_attention_walk_kernel<true>, dim3(blocks, (nc + p.cpb - 1) / p.cpb),
-                           dim3(kPaWaves * kWave), 0, s, p);
+        hipLaunchKernelGGL(prefill_attention_walk_kernel<true>, dim3(g.blocks, g.splits), dim3(kPaWaves * kWave), 0, s,
+                           p);
         return launch_attention_combine(c, s);
     }
     if (pa_score_bytes(p.p0, p.rows, p.heads) <= p.part_bytes)

@@ -418,6 +418,22 @@ def test_qwen3_4b_prefill_attention_forms(qwen, start, n):
     b.check_status()
 
 
+@pytest.mark.parametrize("heads,kv", [(16, 8), (6, 2), (3, 3), (8, 2)])
+def test_prefill_attention_mixed_blocks(heads, kv):
+    # head counts and starts for which a block's four (tile, head) slots mix
+    # tiles of one chunk and of two (never with four heads per kv head)
+    from harsh4b_amd.synthetic import random_model
+    config = {"hidden_size": 256, "intermediate_size": 512, "num_attention_heads": heads, "num_key_value_heads": kv,
+              "head_dim": 128, "num_hidden_layers": 2, "vocab_size": 515, "rms_norm_eps": 1e-6,
+              "rope_theta": 1000000, "max_position_embeddings": 1024}
+    model = random_model(config, 5, dev())
+    rng = np.random.default_rng(heads)
+    for start in (16, 20, 33, 48, 60):
+        earlier = [int(t) for t in rng.integers(0, 515, start)]
+        for n in (45, 60, 300):
+            _prefill_vs_steps(model, [int(t) for t in rng.integers(0, 515, n)], start + n, start_tokens=earlier)
+
+
 def test_qwen3_4b_prefill_attention_scores_computed_twice(qwen):
     # 2000 tokens after 5000: the scores exceed the workspace, so the kernel
     # walks the keys twice; pieces of 300 tokens keep theirs
