@@ -1371,16 +1371,6 @@ hipError_t launch_step_attention(const AttnParams& a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_one_chunk_attention(const AttnParams& a, hipStream_t s)
-{
-    if (a.head_dim != 128 || a.context + a.batch - 1 > kAttnChunk) return hipErrorInvalidValue;
-    if (a.groups <= 4)
-        hipLaunchKernelGGL((attention_kernel<128, 4, false, 1>), dim3(a.kv_heads, 1, a.batch), dim3(kBlock), 0, s, a);
-    else
-        hipLaunchKernelGGL((attention_kernel<128, 8, false, 1>), dim3(a.kv_heads, 1, a.batch), dim3(kBlock), 0, s, a);
-    return hipGetLastError();
-}
-
 hipError_t launch_attention_combine(const AttnParams& a, hipStream_t s)
 {
     if (a.head_dim != 128) return hipErrorInvalidValue;
@@ -1388,6 +1378,16 @@ hipError_t launch_attention_combine(const AttnParams& a, hipStream_t s)
     hipLaunchKernelGGL((attention_combine_kernel<128, false>), dim3((a.kv_heads * a.groups + hpb - 1) / hpb, a.batch),
                        dim3(kBlock), 0, s, a);
     return hipGetLastError();
+}
+
+hipError_t launch_query_attention(const AttnParams& a, hipStream_t s)
+{
+    if (a.head_dim != 128 || a.context + a.batch - 1 > a.max_chunks * kAttnChunk) return hipErrorInvalidValue;
+    const dim3 grid(a.kv_heads, a.max_chunks, a.batch);
+    if (a.groups <= 4) hipLaunchKernelGGL((attention_kernel<128, 4, false, 1>), grid, dim3(kBlock), 0, s, a);
+    else hipLaunchKernelGGL((attention_kernel<128, 8, false, 1>), grid, dim3(kBlock), 0, s, a);
+    if (a.max_chunks == 1) return hipGetLastError();
+    return launch_attention_combine(a, s);
 }
 
 }  // namespace hq

@@ -181,9 +181,10 @@ hipError_t gemm_run(const int8_t* x, const float* act, const uint8_t* w, const f
                     int k, char* scratch, hipStream_t s);
 // The decode step's attention (q/k norms, RoPE, K/V write, attention).
 hipError_t launch_step_attention(const AttnParams& a, hipStream_t s);
-// a.batch queries of one chunk at most (query z attends a.context + z
-// positions), one block per query and kv head.
-hipError_t launch_one_chunk_attention(const AttnParams& a, hipStream_t s);
+// a.batch queries (query z attends a.context + z positions, at most
+// a.max_chunks chunks), one block per query, kv head and chunk; the chunk
+// partials of more than one chunk in a.part.
+hipError_t launch_query_attention(const AttnParams& a, hipStream_t s);
 // The combine of the chunk partials in a.part for a.batch queries, query z
 // attending a.context + z positions (one-chunk queries are left alone).
 hipError_t launch_attention_combine(const AttnParams& a, hipStream_t s);

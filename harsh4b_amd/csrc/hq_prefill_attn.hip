@@ -496,9 +496,13 @@ hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s)
     c.max_chunks = nc;
     c.part = p.part;
     c.out = p.out;
-    // one chunk: one query per block fills more of the chip than tiles of 16
-    // (64 tokens: 8.8 us against 14.0)
-    if (nc == 1) return launch_one_chunk_attention(c, s);
+    // One query per block where tiles of 16 leave the chip idle or compute for
+    // absent queries: one chunk (64 tokens: 8.8 us against 14.0), and one or
+    // two queries (hq_prefill over 6 layers of 32 / 8 heads at position 24000:
+    // one query 475 us against 714, two 575 against 719; three are even, four
+    // take 773 against 725).
+    if (nc == 1 || (p.rows <= 2 && pa_part_bytes(p.rows, p.heads, nc) <= p.part_bytes))
+        return launch_query_attention(c, s);
     // fewer blocks than CUs: chunk partials from several blocks per tile, as
     // many as fill two blocks per CU
     if (blocks < 256 && pa_part_bytes(p.rows, p.heads, nc) <= p.part_bytes) {

@@ -434,6 +434,38 @@ def test_prefill_attention_mixed_blocks(heads, kv):
             _prefill_vs_steps(model, [int(t) for t in rng.integers(0, 515, n)], start + n, start_tokens=earlier)
 
 
+@pytest.mark.parametrize("heads,kv", [(16, 8), (8, 2), (2, 2)])
+@pytest.mark.parametrize("start", [61, 62, 64, 700, 4158])
+def test_prefill_of_few_queries(heads, kv, start):
+    # one and two queries (a block per query, head and chunk) and three (tiles
+    # of 16), their contexts on both sides of a chunk edge
+    from harsh4b_amd.synthetic import random_model
+    config = {"hidden_size": 256, "intermediate_size": 512, "num_attention_heads": heads, "num_key_value_heads": kv,
+              "head_dim": 128, "num_hidden_layers": 2, "vocab_size": 515, "rms_norm_eps": 1e-6,
+              "rope_theta": 1000000, "max_position_embeddings": 8192}
+    model = random_model(config, 6, dev())
+    rng = np.random.default_rng(start)
+    for n in (2, 3, 4):                          # the last token goes through the decode step
+        prompt = [int(t) for t in rng.integers(0, 515, n)]
+        a, b = model.new_state(start + n), model.new_state(start + n)
+        for cache in ("keys", "values"):
+            hist = torch.randn((2, start, kv, 128), generator=torch.Generator(dev()).manual_seed(n), device=dev()).half()
+            getattr(a, cache)[:, :start] = hist
+            getattr(b, cache)[:, :start] = hist
+        a.device_position.fill_(start)
+        b.device_position.fill_(start)
+        model.stream.wait_stream(torch.cuda.current_stream())
+        a.position = b.position = start
+        la = to_host(model.prefill(prompt, a)).copy()
+        for t in prompt:
+            lb = model.forward_token(t, b)
+        assert_bits_equal(to_host(a.keys).view(np.uint16), to_host(b.keys).view(np.uint16), f"{n} keys")
+        assert_bits_equal(to_host(a.values).view(np.uint16), to_host(b.values).view(np.uint16), f"{n} values")
+        assert_bits_equal(la, to_host(lb), f"{n} logits")
+        a.check_status()
+        b.check_status()
+
+
 def test_qwen3_4b_prefill_attention_scores_computed_twice(qwen):
     # 2000 tokens after 5000: the scores exceed the workspace, so the kernel
     # walks the keys twice; pieces of 300 tokens keep theirs
