@@ -302,13 +302,34 @@ static bool launch_staged(const GemmParams& p, bool two_groups, hipStream_t s)
     return true;
 }
 
+// Whether 33 to 64 rows take two passes of 32 rather than hq_gemm_tile.hip's
+// tiles.  A pass is one round of blocks while its blocks of 16 outputs are no
+// more than the CUs (n <= 4096; at 4352 outputs it takes 1.2 to 1.5 times as
+// long), the tiles' time is their serial steps of K.  Times of a GEMM in us,
+// passes and tiles, weights from HBM: 33 rows of 2560 x 9728 18.5 and 24.0,
+// of 2560 x 4096 10.7 and 13.8; 64 rows 22.1 and 25.8, 12.2 and 14.0.  Past
+// 4096 columns the passes' blocks have 16 waves and pay off again from 6144
+// columns on (33 rows of 4096 x 6144 17.2 and 18.0; 48 of 4096 x 4608 16.7 and
+// 14.9), with more than 48 rows from 8192 (64 rows of 4096 x 8192 22.4 and
+// 22.7, x 6144 20.3 and 18.9); past 10240 only for few outputs (33 rows of
+// 1024 x 10752 22.4 and 24.2).  Below 1024 columns 64 rows go to the tiles
+// (1024 x 512 8.4 and 8.0).
+static bool two_passes(int m, int n, int k)
+{
+    if (m > 2 * kMaxBatch || (n + 15) / 16 > 256) return false;
+    if (k <= 4096) return m <= 48 || k >= 1024;
+    if (k <= 10240) return k >= (m <= 48 ? 6144 : 8192);
+    return m <= 48 && n <= 2048;
+}
+
 // x: the de-interleaved padded activations.  Wider rows: the kernel with
 // MFMA-shaped weight loads; waves per block: the fewest of 4, 8, 16 whose K
 // ranges fit one round of loads; 32 rows per block from 512 blocks up.
 static hipError_t run_gemm(const int8_t* x, const float* act, const uint8_t* w, const float* ws,
                            float* out, int m, int n, int k, int32_t* acc_out, hipStream_t s)
 {
-    if (m > kMaxBatch && gemm_tile_fits(m, n, k)) return gemm_tile_run(x, act, w, ws, out, m, n, k, acc_out, s);
+    if (m > kMaxBatch && gemm_tile_fits(m, n, k) && !two_passes(m, n, k))
+        return gemm_tile_run(x, act, w, ws, out, m, n, k, acc_out, s);
     const int kp = padded_k(k);
     const int nds = (k + 127) / 128;
     const int waves = nds <= 4 * 6 ? 4 : nds <= 8 * 6 ? 8 : 16;

@@ -412,6 +412,25 @@ def test_batched_gemm_tiles(m, rows, width):
     assert_bits_equal(to_host(out), (ref.astype(np.float32) * a[:, None]) * s[None, :], "out")
 
 
+@pytest.mark.parametrize("m,rows,width", [(33, 4096, 1024), (33, 4097, 1024), (49, 130, 992), (48, 70, 992),
+                                          (48, 100, 6144), (49, 100, 6144), (64, 100, 8192), (64, 70, 8160),
+                                          (64, 4096, 4096), (64, 40, 4128), (65, 70, 4096), (48, 40, 10272),
+                                          (34, 2049, 10272)])
+def test_batched_gemm_between_passes_and_tiles(m, rows, width):
+    # 33 to 64 rows: two passes of 32 rows and the tiles, at the edges of the rule
+    ls = lightspark()
+    rng = np.random.default_rng(m + 3 * rows + width)
+    packed = oracle.pack_int4(random_int4(rng, rows, width))
+    s = rng.uniform(0.005, 0.02, rows).astype(np.float32)
+    q = rng.integers(-127, 128, (m, width)).astype(np.int8)
+    a = rng.uniform(0.001, 0.01, m).astype(np.float32)
+    acc = torch.empty((m, rows), dtype=torch.int32, device=dev())
+    out = ls.int4_i8_gemm(to_dev(q), to_dev(a), ls.LiteSparkProjection(to_dev(packed), to_dev(s)), acc_out=acc)
+    ref = oracle.int4_i8_gemm_acc(q, packed, rows, width)
+    assert_bits_equal(to_host(acc), ref, "acc")
+    assert_bits_equal(to_host(out), (ref.astype(np.float32) * a[:, None]) * s[None, :], "out")
+
+
 @pytest.mark.parametrize("kv,g,d,ctx", [(2, 1, 16, 4097), (1, 8, 32, 8257), (2, 5, 64, 8193), (2, 4, 128, 33000),
                                         (1, 7, 128, 33089)])
 def test_gqa_long_contexts(kv, g, d, ctx):
