@@ -8,8 +8,8 @@
 //           o[d] = fmaf chain of e_t * v_t[d] over ascending t;
 //   combine M = max m_c; a_c = exp(m_c - M); L and O[d] as fmaf chains over
 //           ascending c; out = O * (1 / L).
-// Contexts of up to flash_chunks chunks run in one latency-bound launch
-// (gqa_flash_kernel); longer ones as a memory-bound launch over the chunks
+// Short contexts run in one latency-bound launch (gqa_flash_kernel; the rule
+// is one_launch's); longer ones as a memory-bound launch over the chunks
 // and a combine (gqa_items_kernel, gqa_combine_kernel).
 #include <algorithm>
 #include <mutex>
@@ -716,18 +716,28 @@ static hipError_t launch_items(const GqaParams& a, hipStream_t s)
 }
 
 // The one-launch kernel while one combine batch holds every chunk (4096
-// positions of 8 x 4 heads: 11.6 us against 13; 8192: 20.7 against 18.1,
-// 32767: 66 against 40.6), and up to two batches with more than four query
-// heads per kv head (4 x 8 heads, 8192: 17.8 against 18.1, 16384: 31 against
-// 22).
-static int flash_chunks(int groups) { return groups <= 4 ? kFlashCB : 2 * kFlashCB; }
+// positions of 8 x 4 heads of 128: 11.6 us against 13).  Up to two batches
+// with more than four query heads per kv head (4 x 8 heads, 8192: 17.2
+// against 18.1, 16384: 31 against 22), and for heads of 128 where the items'
+// launch gains little from its waves: up to 512 of them (2 x 4 heads, 8192:
+// 13.3 against 14.9; 4 x 4, 4097: 13.1 against 15.1; 8192, 512 items: 15.1
+// against 15.4; but 8 x 4, 4608, 576 items: 16.5 against 15.9), and just past
+// one block of four a CU, where some CUs take two (16 x 4 heads, 4097, 1040
+// items: 20.8 against 22.2; 5120, 1280: 22.9 against 23.6; 8192, 2048: 30.2
+// against 27.4; 8 x 4, 8192, 1024: 20.8 against 18.4).
+static bool one_launch(int nc, int kv_heads, int groups, int head_dim)
+{
+    if (nc <= kFlashCB || nc > 2 * kFlashCB) return nc <= kFlashCB;
+    const int items = nc * kv_heads;
+    return groups > 4 || (head_dim == 128 && (items <= 512 || (items > 1024 && items <= 1280)));
+}
 
 // head_dim 16/32/64/128, groups <= 8 (checked by the caller)
 static hipError_t launch_gqa_decode(const float* query, const uint16_t* keys, const uint16_t* values, uint32_t* words,
                                     float* output, int context, int kv_heads, int groups, int head_dim, hipStream_t s)
 {
     const int nc = (context + kAttnChunk - 1) / kAttnChunk;
-    if (nc <= flash_chunks(groups)) {
+    if (one_launch(nc, kv_heads, groups, head_dim)) {
         FlashParams a{};
         a.q = query;
         a.keys = keys;

@@ -450,6 +450,24 @@ def test_gqa_long_contexts(kv, g, d, ctx):
         assert_bits_equal(to_host(out), np.asarray(ref).reshape(kv * g, d), f"context {n}")
 
 
+@pytest.mark.parametrize("kv,g,d,ctx", [(4, 2, 128, 8192), (4, 1, 128, 8193), (8, 1, 128, 4097), (8, 2, 128, 8192),
+                                        (16, 1, 128, 4097), (16, 2, 128, 5121), (1, 4, 128, 8192), (8, 4, 64, 4160)])
+def test_gqa_one_launch_and_two(kv, g, d, ctx):
+    # both sides of the rule between the one-launch kernel (two combine
+    # batches) and the items and combine launches
+    ls = lightspark()
+    rng = np.random.default_rng(ctx + kv)
+    q = rng.standard_normal((kv * g, d)).astype(np.float32)
+    k = rng.standard_normal((ctx, kv, d)).astype(np.float16)
+    v = rng.standard_normal((ctx, kv, d)).astype(np.float16)
+    qd, kd, vd = to_dev(q), to_dev(k), to_dev(v)
+    out = torch.empty((kv * g, d), dtype=torch.float32, device=dev())
+    for n in (ctx, ctx - 1, 70, ctx):
+        ls.gqa_decode(qd, kd, vd, out, n, kv, g, d)
+        ref = oracle.gqa_decode_split(q, k[:n].view(np.uint16), v[:n].view(np.uint16), n, kv, g, d)
+        assert_bits_equal(to_host(out), np.asarray(ref).reshape(kv * g, d), f"context {n}")
+
+
 @pytest.mark.parametrize("n,top_k", [(151936, 65), (151936, 256), (151936, 257), (9000, 1365), (20481, 1366),
                                      (12289, 2048), (8192, 129), (300, 300), (130, 2048)])
 @pytest.mark.parametrize("flat", [False, True])
