@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kBlock) void prefill_qk_kernel(QkParams p)
 
 __global__ void prefill_position_kernel(int32_t* position, int value) { *position = value; }
 
-// Workspace layout for a model and KV capacity.
+// Workspace layout for calls that end within `capacity` positions.
 struct PrefillLayout {
     size_t x, q8, act, qkv, qh, att, proj, gu, gemm, part, attn_part, total;
     int kp, qkv_rows, qd;
@@ -337,11 +337,14 @@ static PrefillLayout prefill_layout(const hq_model* m, int capacity)
     L.x = take(size_t(B) * H * 4);
     L.q8 = take(size_t(gemm_padded_m(B)) * L.kp);
     L.act = take(size_t(B) * 4);
+    // the gate and up rows (of up to 32 tokens), or their SwiGLU (hq_prefill),
+    // follow the attention and lie in the place of qkv and the rotated queries
+    L.gu = off;
     L.qkv = take(size_t(B) * L.qkv_rows * 4);
     L.qh = take(size_t(B) * L.qd * 4);
+    off = std::max(off, L.gu + al256p(std::max(size_t(B) * I, size_t(std::min(B, 32)) * 2 * I) * 4));
     L.att = take(size_t(B) * L.qd * 4);
     L.proj = take(size_t(B) * H * 4);
-    L.gu = take(size_t(B) * 2 * I * 4);
     size_t g = gemm_scratch_bytes(B, L.qkv_rows, H);
     g = std::max<size_t>(g, gemm_scratch_bytes(B, H, L.qd));
     g = std::max<size_t>(g, gemm_scratch_bytes(B, 2 * I, H));
@@ -640,7 +643,7 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
     if (reinterpret_cast<uintptr_t>(workspace) & 255u) return HQ_ERR_ALIGN;
     if (count == 0) return HQ_OK;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const PrefillLayout L = prefill_layout(m, st->capacity);
+    const PrefillLayout L = prefill_layout(m, start + count);
     char* ws = static_cast<char*>(workspace);
     float* x = reinterpret_cast<float*>(ws + L.x);
     int8_t* q8 = reinterpret_cast<int8_t*>(ws + L.q8);
@@ -715,7 +718,7 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
             a.values = qp.values;
             a.out = att;
             a.part = reinterpret_cast<float*>(ws + L.attn_part);
-            a.part_bytes = prefill_attention_part_bytes(std::min(kPrefillBatch, st->capacity), m->heads, st->capacity);
+            a.part_bytes = L.total - L.attn_part;
             a.time_stride = time_stride;
             a.p0 = p0;
             a.rows = rows;
@@ -737,7 +740,7 @@ extern "C" int hq_prefill(const hq_model* m, const hq_state* st, const int32_t* 
             if ((e = run_rows(ROW_RESID_NORM, rp, rows, s))) return e;
             // SwiGLU (in the tiled GEMM's epilogue where it writes whole
             // sums), down (its residual is added at the next layer's input)
-            const bool fused = rows > 32 && gemm_part_splits(rows, 2 * I, H) == 0 && gemm_tile_fits(rows, 2 * I, H);
+            const bool fused = rows > 32 && gemm_part_splits(rows, 2 * I, H) == 0;
             rp.sums = GemmSums{};
             const hipError_t ge = fused ? gemm_tile_swiglu(q8, act, Ly.gate_up, Ly.gate_up_scales, gu, rows, I, H, s)
                                         : project(Ly.gate_up, Ly.gate_up_scales, gu, 2 * I, H, rp.sums);

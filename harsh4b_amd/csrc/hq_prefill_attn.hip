@@ -315,12 +315,6 @@ __device__ __forceinline__ void pa_store_out(const PrefillAttnParams& p, const P
     }
 }
 
-// Chunks of the tiles before `tile` (tile i has i / 4 + 1).
-__host__ __device__ constexpr size_t pa_chunks_before(int tile)
-{
-    const size_t a = size_t(tile) / 4, b = size_t(tile) % 4;
-    return 2 * a * (a + 1) + b * (a + 1);
-}
 constexpr int kPaScoreVecs = kAttnChunk * kPaTile / 4;   // float4s of a tile's scores for one chunk and head
 
 // A pass over the keys that writes each chunk's masked scores to the
@@ -336,7 +330,7 @@ __global__ __launch_bounds__(kPaWaves * kWave, 3) void prefill_attention_kernel(
     const int nb = w.nc_block;
     pa_copy<true>(p, w, 0, lds[0]);
     float4* sc = reinterpret_cast<float4*>(p.part) +
-                 ((pa_chunks_before(w.tile) - pa_chunks_before(p.p0 / kPaTile)) * size_t(p.heads) +
+                 (size_t(pa_chunks_before(w.tile) - pa_chunks_before(p.p0 / kPaTile)) * size_t(p.heads) +
                   size_t(w.h) * size_t(w.nc)) * kPaScoreVecs + lane;
     float M = -__builtin_inff();
     {
@@ -453,27 +447,29 @@ __global__ __launch_bounds__(kPaWaves * kWave, 2) void prefill_attention_walk_ke
     if (w.store && pa_stores_output(PART, w.nc, c_begin)) pa_store_out(p, w, L, oe, oo);
 }
 
-// Workspace limit (larger batches or contexts take the two-pass form, which
-// needs none).
+// Workspace limit: batches whose scores exceed it take the two-pass form,
+// which needs none (2048 tokens of 32 heads up to position 4096 store 805 MB;
+// in two halves of half the blocks they took 1.16 times as long, and more in
+// smaller pieces).
 constexpr size_t kPaPartBytes = size_t(1) << 30;
 
-static size_t pa_part_bytes(size_t rows, int heads, size_t chunks)
+constexpr size_t kPaPartialBytes = size_t(kPaD + 2) * 4;          // a query, head and chunk
+constexpr size_t kPaScoreBytes = size_t(kPaScoreVecs) * 16;       // a tile, head and chunk
+
+static size_t pa_part_bytes(const PrefillAttnParams& p)
 {
-    return rows * size_t(heads) * chunks * size_t(kPaD + 2) * 4;
+    return size_t(pa_partials(pa_batch(p))) * size_t(p.heads) * kPaPartialBytes;
 }
-static size_t pa_score_bytes(int p0, int rows, int heads)
+static size_t pa_score_bytes(const PrefillAttnParams& p)
 {
-    return (pa_chunks_before((p0 + rows - 1) / kPaTile + 1) - pa_chunks_before(p0 / kPaTile)) * size_t(heads) *
-           kPaScoreVecs * 16;
+    return size_t(pa_tile_chunks(pa_batch(p))) * size_t(p.heads) * kPaScoreBytes;
 }
 
 size_t prefill_attention_part_bytes(int rows, int heads, int capacity)
 {
-    // the largest of what any batch of up to `rows` queries inside the cache
-    // may take, within the limit
-    const size_t chunks = (size_t(capacity) + kAttnChunk - 1) / kAttnChunk;
-    const size_t scores = (size_t(rows) / kPaTile + 2) * chunks * size_t(heads) * kPaScoreVecs * 16;
-    return std::min(std::max(pa_part_bytes(rows, heads, chunks), scores), kPaPartBytes);
+    const size_t partials = size_t(pa_max_partials(rows, heads, capacity)) * size_t(heads) * kPaPartialBytes;
+    const size_t scores = size_t(pa_max_tile_chunks(rows, capacity)) * size_t(heads) * kPaScoreBytes;
+    return std::min(std::max(partials, scores), kPaPartBytes);
 }
 
 hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s)
@@ -481,7 +477,6 @@ hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s)
     if (a.rows < 1 || a.p0 < 0 || a.groups < 1 || a.groups > 8) return hipErrorInvalidValue;
     PrefillAttnParams p = a;
     p.heads = a.kv_heads * a.groups;
-    const int blocks = pa_blocks_per_kv(pa_batch(p)) * p.kv_heads;
     const int nc = (p.p0 + p.rows - 1) / kAttnChunk + 1;
     AttnParams c{};
     c.q = p.q;
@@ -501,11 +496,11 @@ hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s)
     // two queries (hq_prefill over 6 layers of 32 / 8 heads at position 24000:
     // one query 475 us against 714, two 575 against 719; three are even, four
     // take 773 against 725).
-    if (nc == 1 || (p.rows <= 2 && pa_part_bytes(p.rows, p.heads, nc) <= p.part_bytes))
+    if (nc == 1 || (p.rows <= 2 && pa_part_bytes(p) <= p.part_bytes))
         return launch_query_attention(c, s);
     // fewer blocks than CUs: chunk partials from several blocks per tile, as
     // many as fill two blocks per CU
-    if (blocks < 256 && pa_part_bytes(p.rows, p.heads, nc) <= p.part_bytes) {
+    if (pa_takes_partials(pa_batch(p)) && pa_part_bytes(p) <= p.part_bytes) {
         const PaPartGrid g = pa_part_grid(pa_batch(p));
         p.cpb = g.cpb;
         p.part_chunks = nc;
@@ -513,7 +508,8 @@ hipError_t launch_prefill_attention(const PrefillAttnParams& a, hipStream_t s)
                            p);
         return launch_attention_combine(c, s);
     }
-    if (pa_score_bytes(p.p0, p.rows, p.heads) <= p.part_bytes)
+    const int blocks = pa_blocks_per_kv(pa_batch(p)) * p.kv_heads;
+    if (pa_score_bytes(p) <= p.part_bytes)
         hipLaunchKernelGGL(prefill_attention_kernel, dim3(blocks), dim3(kPaWaves * kWave), 0, s, p);
     else
         hipLaunchKernelGGL(prefill_attention_walk_kernel<false>, dim3(blocks), dim3(kPaWaves * kWave), 0, s, p);

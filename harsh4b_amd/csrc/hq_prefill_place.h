@@ -63,6 +63,38 @@ constexpr PaPartGrid pa_part_grid(const PaBatch& b)
     return PaPartGrid{blocks, (nc + cpb - 1) / cpb, cpb};
 }
 
+// Chunks of the tiles before `tile` (tile i has i / 4 + 1).
+constexpr long long pa_chunks_before(int tile)
+{
+    const long long a = tile / 4, b = tile % 4;
+    return 2 * a * (a + 1) + b * (a + 1);
+}
+
+// What a batch's launch keeps in the workspace, per head: chunk partials (of
+// every query and chunk) below kPaCUs blocks, else scores (of every tile and
+// chunk).
+constexpr bool pa_takes_partials(const PaBatch& b) { return pa_blocks_per_kv(b) * b.kv_heads < kPaCUs; }
+constexpr long long pa_partials(const PaBatch& b) { return (long long)b.rows * ((b.p0 + b.rows - 1) / kPaChunk + 1); }
+constexpr long long pa_tile_chunks(const PaBatch& b)
+{
+    return pa_chunks_before(b.p0 / kPaTile + pa_tiles(b)) - pa_chunks_before(b.p0 / kPaTile);
+}
+
+// The most of either over all batches of up to `rows` queries in a cache of
+// `capacity` positions; neither falls as the capacity grows.  Partials: a
+// launch below kPaCUs blocks has fewer than kPaCUs * kPaWaves (tile, head)
+// slots.  Scores: the cache's last tiles (a batch may begin inside one).
+constexpr long long pa_max_partials(int rows, int heads, int capacity)
+{
+    const int chunks = (capacity + kPaChunk - 1) / kPaChunk;
+    return (long long)pa_min(rows, (kPaCUs * kPaWaves / heads + 1) * kPaTile) * chunks;
+}
+constexpr long long pa_max_tile_chunks(int rows, int capacity)
+{
+    const int end = (capacity + kPaTile - 1) / kPaTile;
+    return pa_chunks_before(end) - pa_chunks_before(end - pa_min(end, (rows + kPaTile - 1) / kPaTile + 1));
+}
+
 // Whether a wave stores its queries' outputs at the end of its chunks, which
 // begin at c_begin.  Beside partials (part) only one-chunk tiles have outputs
 // to store, in the block that took their chunk: a block's slots may mix tiles

@@ -188,7 +188,6 @@ class QwenDecodeState:
         s.workspace = self.workspace.data_ptr()
         self.struct = s
         self._graphs = {}          # steps -> captured graph of that many greedy steps
-        self._prefill_ws = None
 
     def synchronize(self) -> None:
         self.stream.synchronize()
@@ -342,16 +341,20 @@ class LiteSparkQwen:
         head = ids[:-1]
         if head.size:
             lib = _native.lib()
-            if state._prefill_ws is None:
-                nbytes = lib.hq_prefill_workspace_bytes(ctypes.byref(self.struct), state.capacity)
-                if nbytes == 0:
-                    raise ValueError("model shape is not supported by the batched prefill")
-                state._prefill_ws = torch.zeros(nbytes, dtype=torch.uint8, device=self.device)
-            state.stream.wait_stream(torch.cuda.current_stream(self.device))   # the workspace's zero fill
+            # Scratch for this call alone, on the states' common stream: the
+            # allocator hands it to the next prompt.  Sized by the prompt's
+            # end, in steps of a power of two so that a growing chat finds it again.
+            end = state.position + int(head.size)
+            nbytes = lib.hq_prefill_workspace_bytes(ctypes.byref(self.struct),
+                                                    min(state.capacity, 1 << (end - 1).bit_length()))
+            if nbytes == 0:
+                raise ValueError("model shape is not supported by the batched prefill")
+            state.stream.wait_stream(torch.cuda.current_stream(self.device))
             with torch.cuda.stream(state.stream):
+                workspace = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
                 dev_ids = torch.from_numpy(head.astype(np.int32)).to(self.device)
             check(lib.hq_prefill(ctypes.byref(self.struct), ctypes.byref(state.struct), dev_ids.data_ptr(),
-                                 int(head.size), int(state.position), state._prefill_ws.data_ptr(),
+                                 int(head.size), int(state.position), workspace.data_ptr(),
                                  state.stream.cuda_stream), "hq_prefill")
             dev_ids.record_stream(state.stream)
             state.position += int(head.size)

@@ -252,7 +252,11 @@ int hq_decode_step(const hq_model* model, const hq_state* state, void* stream);
  * write.  No logits are computed: forward the prompt's last token with
  * hq_decode_step.  Leaves *state->position = start + count.  Bad token IDs
  * set HQ_STEP_BAD_TOKEN.  `workspace`: hq_prefill_workspace_bytes(model,
- * state->capacity) bytes, 256-byte aligned, zero-filled before first use.
+ * start + count) bytes or more (the size never falls as its second argument
+ * grows, so state->capacity serves every call), 256-byte aligned, of any
+ * contents: nothing in it outlives the call, so prompts of several states
+ * that follow one another on a stream can share one.  For the 4B shape 12.6
+ * MB up to position 64, 445 MB up to 2048, 1.2 GB at most.
  * Reference counterpart: the token-by-token prompt loop of
  * cpu_lightspark.py:809-810 and inference_runtime.py:177-181. */
 size_t hq_prefill_workspace_bytes(const hq_model* model, int capacity);

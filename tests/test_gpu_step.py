@@ -466,6 +466,41 @@ def test_prefill_of_few_queries(heads, kv, start):
         b.check_status()
 
 
+def test_prefill_scratch_is_not_held_and_needs_no_clearing():
+    # a prompt leaves no memory allocated with its state, gives the same bits
+    # in a workspace of any contents, and stays within the bytes asked for
+    import ctypes
+
+    from harsh4b_amd import _native
+    from harsh4b_amd.synthetic import random_model
+    config = {"hidden_size": 352, "intermediate_size": 3232, "num_attention_heads": 6, "num_key_value_heads": 2,
+              "head_dim": 128, "num_hidden_layers": 2, "vocab_size": 515, "rms_norm_eps": 1e-6,
+              "rope_theta": 1000000, "max_position_embeddings": 1024}
+    model = random_model(config, 4, dev())
+    lib = _native.lib()
+    rng = np.random.default_rng(4)
+    for n in (3, 20, 33, 65, 130, 600):
+        prompt = [int(t) for t in rng.integers(0, 515, n)]
+        a, b = model.new_state(700), model.new_state(700)
+        torch.cuda.synchronize()
+        held = torch.cuda.memory_allocated()
+        model.prefill(prompt, a)
+        torch.cuda.synchronize()
+        assert torch.cuda.memory_allocated() == held
+        nbytes = lib.hq_prefill_workspace_bytes(ctypes.byref(model.struct), n - 1)
+        ws = torch.full((nbytes + 65536,), 0xFF, dtype=torch.uint8, device=dev())   # (NaN as floats)
+        ids = to_dev(np.array(prompt[:-1], np.int32))
+        torch.cuda.synchronize()
+        assert lib.hq_prefill(ctypes.byref(model.struct), ctypes.byref(b.struct), ids.data_ptr(), n - 1, 0,
+                              ws.data_ptr(), model.stream.cuda_stream) == 0
+        b.position = n - 1
+        lb = to_host(model.forward_token(prompt[-1], b))
+        assert bool((ws[nbytes:] == 0xFF).all())
+        assert_bits_equal(to_host(a.logits), lb, f"{n} logits")
+        assert_bits_equal(to_host(a.keys).view(np.uint16), to_host(b.keys).view(np.uint16), f"{n} keys")
+        assert_bits_equal(to_host(a.values).view(np.uint16), to_host(b.values).view(np.uint16), f"{n} values")
+
+
 def test_qwen3_4b_prefill_attention_scores_computed_twice(qwen):
     # 2000 tokens after 5000: the scores exceed the workspace, so the kernel
     # walks the keys twice; pieces of 300 tokens keep theirs
