@@ -33,3 +33,12 @@ def assert_bits_equal(actual, expected, what=""):
         i = bad[0]
         raise AssertionError(f"{what}: {bad.size} of {a.size} differ; first at {i}: "
                              f"{a.ravel()[i]!r} vs {e.ravel()[i]!r}")
+
+
+def assert_bits_or_nan_equal(actual, expected, what=""):
+    """Equal bits, but any NaN for a NaN (its sign and payload are free)."""
+    a, e = (np.array(x, copy=True) for x in (actual, expected))
+    assert a.shape == e.shape, (what, a.shape, e.shape)
+    a[np.isnan(a)] = np.nan
+    e[np.isnan(e)] = np.nan
+    assert_bits_equal(a, e, what)

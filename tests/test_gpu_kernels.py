@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from tests.gpu_util import assert_bits_equal, dev, random_int4, to_dev, to_host
+from tests.gpu_util import assert_bits_equal, assert_bits_or_nan_equal, dev, random_int4, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -466,6 +466,44 @@ def test_gqa_one_launch_and_two(kv, g, d, ctx):
         ls.gqa_decode(qd, kd, vd, out, n, kv, g, d)
         ref = oracle.gqa_decode_split(q, k[:n].view(np.uint16), v[:n].view(np.uint16), n, kv, g, d)
         assert_bits_equal(to_host(out), np.asarray(ref).reshape(kv * g, d), f"context {n}")
+
+
+@pytest.mark.parametrize("kv,g,d,n", [(8, 4, 128, 300), (8, 4, 128, 64), (2, 4, 128, 5000), (8, 4, 128, 4999),
+                                      (8, 3, 128, 9000), (1, 8, 64, 9000), (2, 2, 16, 4161)])
+def test_gqa_infinities_and_nan(kv, g, d, n):
+    # rows past the context hold infinities and NaN; then scores of -inf (single
+    # positions, a whole chunk), values of +-inf and NaN at a few positions
+    # inside it: one launch, two combine batches, and the items' launch
+    ls = lightspark()
+    rng = np.random.default_rng(n + d)
+    cap = n + 70
+    q = np.abs(rng.standard_normal((kv * g, d))).astype(np.float32)      # (a key of -inf scores -inf)
+    k = rng.standard_normal((cap, kv, d)).astype(np.float16)
+    v = rng.standard_normal((cap, kv, d)).astype(np.float16)
+    k[n:] = np.inf
+    v[n:] = np.nan
+    out = torch.empty((kv * g, d), dtype=torch.float32, device=dev())
+
+    def check(what):
+        ls.gqa_decode(to_dev(q), to_dev(k), to_dev(v), out, n, kv, g, d)
+        ref = oracle.gqa_decode_split(q, k[:n].view(np.uint16), v[:n].view(np.uint16), n, kv, g, d)
+        ref = np.asarray(ref).reshape(kv * g, d)
+        assert_bits_or_nan_equal(to_host(out), ref, what)
+        return ref
+
+    assert np.isfinite(check("unseen rows")).all()
+    k[n - 2, 0, 3] = -np.inf
+    k[n // 2, :, d - 1] = -np.inf
+    assert np.isfinite(check("scores of -inf")).all()
+    v[n // 3, 0, 5] = np.inf
+    v[n - 2, kv - 1, 0] = -np.inf
+    v[0, 0, 1] = np.nan
+    check("infinite values")
+    k[0:min(64, n), 0, 0] = -np.inf
+    check("a chunk of -inf")
+    k[n // 4, kv - 1, 1] = np.inf
+    k[n // 5, 0, 2] = np.nan
+    check("scores of inf and NaN")
 
 
 @pytest.mark.parametrize("n,top_k", [(151936, 65), (151936, 256), (151936, 257), (9000, 1365), (20481, 1366),

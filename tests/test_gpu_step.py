@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 import oracle
-from tests.gpu_util import assert_bits_equal, dev, to_dev, to_host
+from tests.gpu_util import assert_bits_equal, assert_bits_or_nan_equal, dev, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -376,8 +376,8 @@ def test_tiny_model_prefill_flags_bad_tokens(forward_golden):
 
 
 def test_qwen3_4b_prefill_matches_token_steps(qwen):
-    # 200 tokens: two batches of the prefill (128 + 71), contexts up to four
-    # attention splits, the layer kernel for the comparison steps
+    # 200 tokens after two: contexts of up to four chunks, the layer kernel for
+    # the comparison steps
     model, _ = qwen
     rng = np.random.default_rng(21)
     prompt = [int(t) for t in rng.integers(0, 151936, 200)]
@@ -386,7 +386,7 @@ def test_qwen3_4b_prefill_matches_token_steps(qwen):
 
 def test_qwen3_4b_prefill_after_a_long_turn(qwen):
     # a 300-token prompt after a 300-token earlier turn: query contexts 301-600
-    # (up to ten chunks, three attention splits), three prefill batches
+    # (up to ten chunks)
     model, _ = qwen
     rng = np.random.default_rng(33)
     earlier = [int(t) for t in rng.integers(0, 151936, 300)]
@@ -466,6 +466,82 @@ def test_prefill_of_few_queries(heads, kv, start):
         b.check_status()
 
 
+@pytest.mark.parametrize("heads,kv,start,n", [(16, 8, 20, 100), (16, 8, 200, 3), (8, 2, 200, 150), (16, 8, 200, 1100),
+                                              (3, 3, 130, 40)])
+def test_prefill_attention_infinities_and_nan(heads, kv, start, n):
+    # cache rows past the prompt hold infinities and NaN; then keys of huge
+    # values, and in the second of three layers values of +-inf and NaN and an
+    # infinite key: chunk partials and (1100 tokens) stored scores against
+    # pieces of two tokens, which take one query per block
+    import ctypes
+
+    from harsh4b_amd import _native
+    from harsh4b_amd.synthetic import random_model
+    config = {"hidden_size": 256, "intermediate_size": 512, "num_attention_heads": heads, "num_key_value_heads": kv,
+              "head_dim": 128, "num_hidden_layers": 3, "vocab_size": 515, "rms_norm_eps": 1e-6,
+              "rope_theta": 1000000, "max_position_embeddings": 2048}
+    model = random_model(config, 7, dev())
+    lib = _native.lib()
+    rng = np.random.default_rng(start + n)
+    ids = to_dev(rng.integers(0, 515, n).astype(np.int32))
+    ws = torch.empty(lib.hq_prefill_workspace_bytes(ctypes.byref(model.struct), start + n), dtype=torch.uint8,
+                     device=dev())
+    for infinite in (False, True):
+        states = [model.new_state(start + n + 80) for _ in range(2)]
+        for st in states:
+            for cache in (st.keys, st.values):
+                gen = torch.Generator(device=dev()).manual_seed(9)
+                cache[:, :start] = torch.randn((3, start, kv, 128), generator=gen, device=dev()).half()
+            st.keys[:, start // 2, 0, 7] = 60000.0
+            st.keys[:, start - 1, kv - 1, 100] = -60000.0
+            if infinite:
+                st.values[1, start // 3, 0, 5] = float("inf")
+                st.values[1, start - 2, kv - 1, 0] = float("-inf")
+                st.values[1, 0, 0, 1] = float("nan")
+                st.keys[1, 1, 0, 3] = float("inf")
+            st.keys[:, start + n:] = float("inf")
+            st.values[:, start + n:] = float("nan")
+        torch.cuda.synchronize()
+        for st, piece in zip(states, (n, 2)):
+            for i in range(0, n, piece):
+                assert lib.hq_prefill(ctypes.byref(model.struct), ctypes.byref(st.struct), ids[i:].data_ptr(),
+                                      min(piece, n - i), start + i, ws.data_ptr(), model.stream.cuda_stream) == 0
+        for name in ("keys", "values"):
+            x, y = (to_host(getattr(st, name))[:, :start + n].astype(np.float32) for st in states)
+            assert_bits_or_nan_equal(x, y, f"{name} infinite={infinite}")
+            assert infinite or np.isfinite(x).all()
+
+
+@pytest.mark.parametrize("heads,kv,start,n", [(16, 8, 5, 2060), (6, 2, 0, 4200), (32, 8, 201, 1100), (16, 8, 1000, 1300)])
+def test_prefill_passes_and_stored_scores(heads, kv, start, n):
+    # prompts of two and three passes of 2048 tokens, each with its own first
+    # position, and stored scores of tiles that begin inside one past position 0
+    from harsh4b_amd.synthetic import random_model
+    config = {"hidden_size": 256, "intermediate_size": 512, "num_attention_heads": heads, "num_key_value_heads": kv,
+              "head_dim": 128, "num_hidden_layers": 2, "vocab_size": 515, "rms_norm_eps": 1e-6,
+              "rope_theta": 1000000, "max_position_embeddings": 8192}
+    model = random_model(config, 8, dev())
+    rng = np.random.default_rng(n)
+    _prefill_vs_steps(model, [int(t) for t in rng.integers(0, 515, n)], start + n,
+                      start_tokens=[int(t) for t in rng.integers(0, 515, start)])
+
+
+def test_qwen3_4b_prefill_of_two_passes(qwen):
+    # 2300 tokens in one call (2048 + 251) and in pieces within a pass
+    model, _ = qwen
+    rng = np.random.default_rng(2300)
+    prompt = [int(t) for t in rng.integers(0, 151936, 2300)]
+    a, b = model.new_state(2300), model.new_state(2300)
+    la = to_host(model.prefill(prompt, a)).copy()
+    for i in range(0, 2300, 900):
+        lb = model.prefill(prompt[i:i + 900], b)
+    assert_bits_equal(la, to_host(lb), "logits")
+    assert_bits_equal(to_host(a.keys).view(np.uint16), to_host(b.keys).view(np.uint16), "keys")
+    assert_bits_equal(to_host(a.values).view(np.uint16), to_host(b.values).view(np.uint16), "values")
+    a.check_status()
+    b.check_status()
+
+
 def test_prefill_scratch_is_not_held_and_needs_no_clearing():
     # a prompt leaves no memory allocated with its state, gives the same bits
     # in a workspace of any contents, and stays within the bytes asked for
@@ -503,7 +579,7 @@ def test_prefill_scratch_is_not_held_and_needs_no_clearing():
 
 def test_qwen3_4b_prefill_attention_scores_computed_twice(qwen):
     # 2000 tokens after 5000: the scores exceed the workspace, so the kernel
-    # walks the keys twice; pieces of 300 tokens keep theirs
+    # walks the keys twice; pieces of 300 tokens write chunk partials
     model, _ = qwen
     rng = np.random.default_rng(5)
     gen = torch.Generator(device=dev()).manual_seed(5)
