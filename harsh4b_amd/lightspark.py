@@ -610,12 +610,15 @@ def _zeroed_workspace(kind: tuple, nbytes: int, device, stream=None) -> torch.Te
     calls on one stream run in order, while calls on two streams may overlap,
     and overlapping calls on one workspace would share its ticket counters.
     The zero fill runs on the current stream; a given `stream` is made to
-    wait for it."""
+    wait for it, and the memory of a workspace outgrown is not reused before
+    the calls that its stream still has on it are done."""
     handle = (stream.cuda_stream if stream is not None
               else torch._C._cuda_getCurrentRawStream(torch.cuda._utils._get_device_index(device)))
     key = (*kind, handle)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
+        if ws is not None:
+            ws.record_stream(stream if stream is not None else torch.cuda.current_stream(device))
         ws = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=device)
         _workspaces[key] = ws
     if stream is not None:

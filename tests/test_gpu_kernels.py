@@ -506,6 +506,30 @@ def test_gqa_infinities_and_nan(kv, g, d, n):
     check("scores of inf and NaN")
 
 
+def test_outgrown_workspace_lives_until_its_calls_are_done():
+    # a call waiting on a side stream, then one there that needs a larger
+    # workspace, then memory of the first one's size filled on the current stream
+    ls = lightspark()
+    rng = np.random.default_rng(12)
+    stream = torch.cuda.Stream()
+    k, v = (rng.standard_normal((4096, 8, 128)).astype(np.float16) for _ in range(2))
+    q = rng.standard_normal((32, 128)).astype(np.float32)
+    qd, kd, vd = to_dev(q), to_dev(k), to_dev(v)
+    small, large = (torch.empty((32, 128), dtype=torch.float32, device=dev()) for _ in range(2))
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(20_000_000)
+    nbytes = ls._gqa_workspace_bytes(512, 8, 4, 128)
+    ls.gqa_decode(qd, kd[:512], vd[:512], small, 512, 8, 4, 128, stream=stream)
+    ls.gqa_decode(qd, kd, vd, large, 4096, 8, 4, 128, stream=stream)
+    filled = [torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=dev()) for _ in range(8)]
+    torch.cuda.synchronize()
+    assert all(bool((f == 0xFF).all()) for f in filled)
+    for out, n in ((small, 512), (large, 4096)):
+        ref = oracle.gqa_decode_split(q, k[:n].view(np.uint16), v[:n].view(np.uint16), n, 8, 4, 128)
+        assert_bits_equal(to_host(out), np.asarray(ref).reshape(32, 128), f"context {n}")
+
+
 @pytest.mark.parametrize("n,top_k", [(151936, 65), (151936, 256), (151936, 257), (9000, 1365), (20481, 1366),
                                      (12289, 2048), (8192, 129), (300, 300), (130, 2048)])
 @pytest.mark.parametrize("flat", [False, True])
