@@ -1,5 +1,6 @@
 // hq_gemm_tile.hip - packed-int4 weights x int8 activation rows for batches
-// of more than 32 rows (prompts): output tiles on v_mfma_i32_32x32x32_i8, the
+// of more than 32 rows (prompts; hq_gemm.hip's two_passes says which of 33 to
+// 64 rows take its kernels twice instead): output tiles on v_mfma_i32_32x32x32_i8, the
 // same integers as hq_gemm.hip's kernels.
 //
 // Activation rows go on the A side (output rows), weight rows on the B side
@@ -283,7 +284,9 @@ template <int EPI>
 static hipError_t run_tile(const TileParams& p, hipStream_t s)
 {
     const long long t = tiles64(p.m, EPI == TILE_SWIGLU ? 2LL * p.n : p.n);
-    if (t <= kSmallTiles) return launch_tile<1, 2, 2, 1, 2, 3, EPI>(p, s);
+    if constexpr (EPI != TILE_SWIGLU) {   // (SwiGLU of so few tiles follows K parts)
+        if (t <= kSmallTiles) return launch_tile<1, 2, 2, 1, 2, 3, EPI>(p, s);
+    }
     if (t <= kMidTiles) return launch_tile<1, 2, 2, 2, 1, 4, EPI>(p, s);
     return launch_tile<2, 2, 2, 2, 1, 2, EPI>(p, s);
 }
@@ -345,7 +348,7 @@ hipError_t gemm_tile_run(const int8_t* x, const float* act, const uint8_t* w, co
 hipError_t gemm_tile_swiglu(const int8_t* x, const float* act, const uint8_t* w, const float* ws, float* out, int m,
                             int n, int k, hipStream_t s)
 {
-    if (!gemm_tile_fits(m, 2 * n, k)) return hipErrorInvalidValue;
+    if (!gemm_tile_fits(m, 2 * n, k) || gemm_part_splits(m, 2 * n, k) != 0) return hipErrorInvalidValue;
     return run_tile<TILE_SWIGLU>(tile_params(x, act, w, ws, out, m, n, k), s);
 }
 
