@@ -508,7 +508,10 @@ __device__ __forceinline__ void gqa_item(const GqaParams& a, uint16_t* ks, int c
 #pragma unroll
     for (int t = 0; t < 32; ++t) v[t] = load_v(t);
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(32)" ::: "memory");   // the K rows (and the queries) are in
+    // the K rows (and the queries) are in: the 32 V loads above are the only
+    // ones issued since (no load crosses the block's memory clobber, nor the
+    // scheduling barriers)
+    asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
 #pragma unroll
     for (int t = 32; t < 64; ++t) v[t] = load_v(t);
     __builtin_amdgcn_sched_barrier(0);

@@ -24,11 +24,16 @@
 // write the chunk partials and let attention_combine_kernel combine them;
 // contexts whose scores exceed the workspace compute them twice.
 //
-// Bound by fp32 arithmetic: the fp32 matrix instructions (256 of 32 cycles per
-// 16 queries, 64 keys and head) and the fp32 vector instructions (about 800
-// of 4 cycles: conversions, tree sums, exponentials) do not run side by side.
-// 2000 tokens of 32 heads: 440 us a layer (1890 us with one query per block
-// on the vector unit, 672 us with the scores computed twice), 75 TFLOP/s.
+// Bound by fp32 arithmetic.  Of the SIMDs' cycles in prefill_attention_kernel
+// the matrix instructions (256 of 32 cycles per 16 queries, 64 keys and head)
+// take 48 % and the other vector instructions (about 1000 of 4 cycles:
+// conversions, tree sums, exponentials) 25 %, by counters; LDS reads conflict
+// in no bank, and memory moves 0.6 GB a layer.  Three waves a SIMD is what the
+// registers allow (168, nine more spilled and reloaded at a chunk's ends, not
+// among its products).
+// 2000 tokens of 32 heads: 440 to 465 us a layer, 70 to 75 TFLOP/s (1890 us
+// with one query per block on the vector unit, 672 us with the scores computed
+// twice).
 #include <algorithm>
 
 #include "hq_device.h"

@@ -27,7 +27,10 @@ constexpr int pa_blocks_per_kv(const PaBatch& b) { return (pa_tiles(b) * b.group
 // (query tile, head) slots of it, the blocks with the longest contexts
 // first -- but the second block of each CU in the opposite order, so that the
 // blocks a CU starts with sum to about the same work (2000 tokens: 72 to 48
-// chunks per wave slot otherwise, 64 to 56 so).
+// chunks per wave slot otherwise, 64 to 56 so).  Four layers of 32 / 8 heads:
+// 1024 tokens 1142 us against 1202, 1500 1713 against 1787, 2000 after 500
+// 3165 against 3329; 2000 from position 0 are even, 1700 after 2000 4443
+// against 4364.
 struct PaSlot {
     int kvh, h, tile, nc, nc_block;   // tile: 16 positions from 16 * tile; nc: its chunks; the block's most
     bool live;                        // (false: the block's last slots repeat another wave's)

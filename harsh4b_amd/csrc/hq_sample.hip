@@ -575,8 +575,9 @@ static size_t al256s(size_t v) { return (v + 255) & ~size_t(255); }
 static int sample_slices(int n) { return (n + kSampleSlice - 1) / kSampleSlice; }
 
 // The counters' fixed place at the workspace's start: calls with any n and k
-// share them.  A tree over up to kSampleNodes slices has fewer nodes than
-// slices; more slices (4.2M logits) merge in one node.
+// share them.  A tree over up to kSampleNodes slices has at most 1023 nodes
+// (lone children can make them more than its slices: 521 over 513); more
+// slices (4.2M logits) merge in one node.
 constexpr int kSampleNodes = 1024;
 constexpr size_t kSampleHead = kSampleNodes * 4;
 

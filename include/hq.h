@@ -256,7 +256,7 @@ int hq_decode_step(const hq_model* model, const hq_state* state, void* stream);
  * grows, so state->capacity serves every call), 256-byte aligned, of any
  * contents: nothing in it outlives the call, so prompts of several states
  * that follow one another on a stream can share one.  For the 4B shape 12.6
- * MB up to position 64, 445 MB up to 2048, 1.2 GB at most.
+ * MiB up to position 64, 445 MiB up to 2048, 1201 MiB at most.
  * Reference counterpart: the token-by-token prompt loop of
  * cpu_lightspark.py:809-810 and inference_runtime.py:177-181. */
 size_t hq_prefill_workspace_bytes(const hq_model* model, int capacity);
