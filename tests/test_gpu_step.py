@@ -512,6 +512,43 @@ def test_prefill_attention_infinities_and_nan(heads, kv, start, n):
             assert infinite or np.isfinite(x).all()
 
 
+@pytest.mark.parametrize("heads,kv,start,n", [(10, 2, 20, 150), (16, 2, 60, 300), (7, 1, 37, 64), (12, 2, 0, 1500)])
+def test_prefill_of_many_heads_per_kv_head(heads, kv, start, n):
+    # five to eight query heads per kv head (the decode step takes up to four,
+    # so the caches are the test's own): tiles against pieces of two tokens
+    import ctypes
+
+    from harsh4b_amd import _native
+    from harsh4b_amd.synthetic import random_model
+    config = {"hidden_size": 256, "intermediate_size": 512, "num_attention_heads": heads, "num_key_value_heads": kv,
+              "head_dim": 128, "num_hidden_layers": 3, "vocab_size": 515, "rms_norm_eps": 1e-6,
+              "rope_theta": 1000000, "max_position_embeddings": 2048}
+    model = random_model(config, 10, dev())
+    lib = _native.lib()
+    rng = np.random.default_rng(n)
+    ids = to_dev(rng.integers(0, 515, n).astype(np.int32))
+    ws = torch.empty(lib.hq_prefill_workspace_bytes(ctypes.byref(model.struct), start + n), dtype=torch.uint8,
+                     device=dev())
+    caches = []
+    for piece in (n, 2):
+        gen = torch.Generator(device=dev()).manual_seed(11)
+        keys, values = (torch.randn((3, start + n, kv, 128), generator=gen, device=dev()).half() for _ in range(2))
+        position, status = (torch.zeros(1, dtype=torch.int32, device=dev()) for _ in range(2))
+        st = _native.HqState()
+        st.capacity = start + n
+        st.keys, st.values = keys.data_ptr(), values.data_ptr()
+        st.position, st.status = position.data_ptr(), status.data_ptr()
+        torch.cuda.synchronize()
+        for i in range(0, n, piece):
+            assert lib.hq_prefill(ctypes.byref(model.struct), ctypes.byref(st), ids[i:].data_ptr(), min(piece, n - i),
+                                  start + i, ws.data_ptr(), model.stream.cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert int(position.item()) == start + n and int(status.item()) == 0
+        caches.append((to_host(keys), to_host(values)))
+    for x, y in zip(*caches):
+        assert_bits_equal(x.view(np.uint16), y.view(np.uint16), f"{heads} / {kv}")
+
+
 @pytest.mark.parametrize("heads,kv,start,n", [(16, 8, 5, 2060), (6, 2, 0, 4200), (32, 8, 201, 1100), (16, 8, 1000, 1300)])
 def test_prefill_passes_and_stored_scores(heads, kv, start, n):
     # prompts of two and three passes of 2048 tokens, each with its own first
