@@ -341,21 +341,26 @@ class LiteSparkQwen:
         head = ids[:-1]
         if head.size:
             lib = _native.lib()
-            # Scratch for this call alone, on the states' common stream: the
-            # allocator hands it to the next prompt.  Sized by the prompt's
-            # end, in steps of a power of two so that a growing chat finds it again.
+            # Scratch for this call alone, from the caller's stream, which waits
+            # for the prompt before its memory is anyone else's.  Sized by the
+            # prompt's end, in steps of a power of two so that a growing chat
+            # finds it again.
             end = state.position + int(head.size)
             nbytes = lib.hq_prefill_workspace_bytes(ctypes.byref(self.struct),
                                                     min(state.capacity, 1 << (end - 1).bit_length()))
             if nbytes == 0:
                 raise ValueError("model shape is not supported by the batched prefill")
-            state.stream.wait_stream(torch.cuda.current_stream(self.device))
+            caller = torch.cuda.current_stream(self.device)
+            workspace = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+            state.stream.wait_stream(caller)
             with torch.cuda.stream(state.stream):
-                workspace = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
                 dev_ids = torch.from_numpy(head.astype(np.int32)).to(self.device)
-            check(lib.hq_prefill(ctypes.byref(self.struct), ctypes.byref(state.struct), dev_ids.data_ptr(),
-                                 int(head.size), int(state.position), workspace.data_ptr(),
-                                 state.stream.cuda_stream), "hq_prefill")
+            try:
+                check(lib.hq_prefill(ctypes.byref(self.struct), ctypes.byref(state.struct), dev_ids.data_ptr(),
+                                     int(head.size), int(state.position), workspace.data_ptr(),
+                                     state.stream.cuda_stream), "hq_prefill")
+            finally:
+                caller.wait_stream(state.stream)
             dev_ids.record_stream(state.stream)
             state.position += int(head.size)
         return self.forward_token(int(ids[-1]), state)

@@ -591,15 +591,20 @@ def test_prefill_scratch_is_not_held_and_needs_no_clearing():
               "rope_theta": 1000000, "max_position_embeddings": 1024}
     model = random_model(config, 4, dev())
     lib = _native.lib()
+    side = torch.cuda.Stream()
     rng = np.random.default_rng(4)
     for n in (3, 20, 33, 65, 130, 600):
         prompt = [int(t) for t in rng.integers(0, 515, n)]
         a, b = model.new_state(700), model.new_state(700)
         torch.cuda.synchronize()
         held = torch.cuda.memory_allocated()
-        model.prefill(prompt, a)
+        with torch.cuda.stream(side):
+            model.prefill(prompt, a)
+            assert torch.cuda.memory_allocated() == held
+            # what reuses the scratch's memory comes after the prompt
+            reused = [torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=dev()) for nbytes in (1 << 20, 4 << 20, 8 << 20)]
         torch.cuda.synchronize()
-        assert torch.cuda.memory_allocated() == held
+        assert all(bool((r == 0xFF).all()) for r in reused)
         nbytes = lib.hq_prefill_workspace_bytes(ctypes.byref(model.struct), n - 1)
         ws = torch.full((nbytes + 65536,), 0xFF, dtype=torch.uint8, device=dev())   # (NaN as floats)
         ids = to_dev(np.array(prompt[:-1], np.int32))
