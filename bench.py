@@ -802,7 +802,7 @@ def attention_case(args, torch, context=4096):
     gbs = nbytes / (us * 1e-6) / 1e9
     del graph, keys, values
     torch.cuda.empty_cache()
-    return {"kernel": "attention_kernel (hq_gqa_decode)", "context": context, "us_per_call": round(us, 3),
+    return {"kernel": "gqa_flash_kernel (hq_gqa_decode)", "context": context, "us_per_call": round(us, 3),
             "algorithmic_bytes": nbytes, "achieved": round(gbs, 1), "unit": "GB/s",
             "frac": round(gbs / HBM_PEAK_GBS, 4)}
 

@@ -31,7 +31,7 @@
 // in no bank, and memory moves 0.6 GB a layer.  Three waves a SIMD is what the
 // registers allow (168, nine more spilled and reloaded at a chunk's ends, not
 // among its products).
-// 2000 tokens of 32 heads: 440 to 465 us a layer, 70 to 75 TFLOP/s (1890 us
+// 2000 tokens of 32 heads: 440 to 480 us a layer by GPU, 68 to 75 TFLOP/s (1890 us
 // with one query per block on the vector unit, 672 us with the scores computed
 // twice).
 #include <algorithm>
