@@ -312,11 +312,13 @@ static bool launch_staged(const GemmParams& p, bool two_groups, hipStream_t s)
 // columns on (33 rows of 4096 x 6144 17.2 and 18.0; 48 of 4096 x 4608 16.7 and
 // 14.9), with more than 48 rows from 8192 (64 rows of 4096 x 8192 22.4 and
 // 22.7, x 6144 20.3 and 18.9); past 10240 only for few outputs (33 rows of
-// 1024 x 10752 22.4 and 24.2).  Below 1024 columns 64 rows go to the tiles
-// (1024 x 512 8.4 and 8.0).
+// 1024 x 10752 22.4 and 24.2).  Up to 256 outputs they do from 4608 columns
+// (33 rows of 64 x 5120 13.3 and 14.5), with more than 48 rows from 6144.
+// Below 1024 columns 64 rows go to the tiles (1024 x 512 8.4 and 8.0).
 static bool two_passes(int m, int n, int k)
 {
     if (m > 2 * kMaxBatch || (n + 15) / 16 > 256) return false;
+    if (k > 4096 && n <= 256) return k >= (m <= 48 ? 4608 : 6144);
     if (k <= 4096) return m <= 48 || k >= 1024;
     if (k <= 10240) return k >= (m <= 48 ? 6144 : 8192);
     return m <= 48 && n <= 2048;

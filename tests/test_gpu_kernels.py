@@ -415,7 +415,8 @@ def test_batched_gemm_tiles(m, rows, width):
 @pytest.mark.parametrize("m,rows,width", [(33, 4096, 1024), (33, 4097, 1024), (49, 130, 992), (48, 70, 992),
                                           (48, 100, 6144), (49, 100, 6144), (64, 100, 8192), (64, 70, 8160),
                                           (64, 4096, 4096), (64, 40, 4128), (65, 70, 4096), (48, 40, 10272),
-                                          (34, 2049, 10272)])
+                                          (34, 2049, 10272), (48, 256, 4608), (33, 257, 4608), (49, 256, 6144),
+                                          (64, 40, 12288)])
 def test_batched_gemm_between_passes_and_tiles(m, rows, width):
     # 33 to 64 rows: two passes of 32 rows and the tiles, at the edges of the rule
     ls = lightspark()
