@@ -727,7 +727,9 @@ static hipError_t launch_items(const GqaParams& a, hipStream_t s)
 // against 15.4; but 8 x 4, 4608, 576 items: 16.5 against 15.9), and just past
 // one block of four a CU, where some CUs take two (16 x 4 heads, 4097, 1040
 // items: 20.8 against 22.2; 5120, 1280: 22.9 against 23.6; 8192, 2048: 30.2
-// against 27.4; 8 x 4, 8192, 1024: 20.8 against 18.4).
+// against 27.4; 8 x 4, 8192, 1024: 20.8 against 18.4).  Heads of 16 to 64 gain
+// nothing from it (of 64, 4097 positions: 2 x 4 12.6 against 13.0, 4 x 4 even,
+// 8 x 4 15.4 against 13.3).
 static bool one_launch(int nc, int kv_heads, int groups, int head_dim)
 {
     if (nc <= kFlashCB || nc > 2 * kFlashCB) return nc <= kFlashCB;
